@@ -48,6 +48,7 @@ void AMGSolver::free_hierarchy()
       l.S.free_all();
       l.Arev.free_all();
       l.ell.free_all();
+      l.sten.free_all();
       l.Av = Csr();
       dfree(l.A32.a32); dfree(l.P32.a32); dfree(l.R32.a32);
       dfree(l.CF); dfree(l.measure); dfree(l.l1); dfree(l.l1f);
@@ -79,10 +80,13 @@ int AMGSolver::sweeps(int lev, int k) const
    return prm.num_sweeps[k];
 }
 
-static void make_fp32_view(const Csr &src, Csr &dst)
+// values: false when only the solve-phase copy's FP32 values are read
+static void make_fp32_view(const Csr &src, Csr &dst, bool values = true)
 {
    dst = src;                 // shares index arrays; owns only a32
    dst.a = nullptr;
+   dst.a32 = nullptr;
+   if (!values) { return; }
    dst.a32 = dalloc_n<float>((size_t) std::max<long long>(src.nnz, 1));
    d2f((int) src.nnz, src.a, dst.a32);
 }
@@ -113,9 +117,34 @@ void AMGSolver::setup(const Csr &A0)
    // A level's copy is filled on the side stream while the level's RAP runs
    // (a latency-bound kernel that leaves HBM bandwidth free), the coarsest
    // level's after the loop.
+   // The fine level gets a stencil copy instead where its rows are those of a
+   // grid stencil; the probe that tells runs beside the first kernels.
    int ell_started = 0;   // levels whose copy is under way
+   bool probed = false;
+   if (p.solve_format == 1) {
+      side_after_main();
+      probed = sten_probe(A0, L[0].sten, 4096, side_stream());
+   }
+   // the full values of the slices that need them, once the fill has said so
+   auto finish_sten = [&]() {
+      if (L[0].sten.nslices <= 0 || L[0].sten.raw) { return; }
+      side_sync();
+      if (sten_raw_slices() > 0) {
+         side_after_main();
+         sten_fill_raw(A0, L[0].sten, p.cycle_fp32 != 0, side_stream());
+      }
+   };
    auto start_ell = [&](int j) {
       Level &lv = L[j];
+      if (j == 0 && probed) {
+         side_sync();
+         if (sten_take(lv.sten)) {
+            side_after_main();
+            sten_fill(A0, lv.sten, side_stream());
+            ell_started = 1;
+            return;
+         }
+      }
       if (p.solve_format == 1 && ell_plan(*lv.A, lv.ell, 0.25, 4096, p.cycle_fp32 != 0)) {
          side_after_main();
          ell_fill(*lv.A, lv.ell, p.cycle_fp32 != 0, side_stream());
@@ -219,6 +248,7 @@ void AMGSolver::setup(const Csr &A0)
       start_ell(level);
       // the copy's plan found the level operator's longest row
       if (a_max_row <= 0 && cur.ell.nslices > 0) { a_max_row = cur.ell.wmax; }
+      if (a_max_row <= 0 && cur.sten.nslices > 0) { a_max_row = cur.sten.tab.wmax; }
       // P's rows: one entry for a C point, at most P_max_elmts otherwise
       const int pmx = aggressive ? p.agg_P_max_elmts : p.P_max_elmts;
       {
@@ -226,6 +256,7 @@ void AMGSolver::setup(const Csr &A0)
          rap(cur.R, *cur.A, cur.P, nx.Aown, pmx > 0 ? std::max(pmx, 1) : 0, a_max_row,
              &a_max_row);
       }
+      if (level == 0) { finish_sten(); }
       nx.A = &nx.Aown;
       level++;
       // par_amg_setup.c:3136-3141 (the host-only switch to CLJP coarsening
@@ -283,7 +314,10 @@ void AMGSolver::setup(const Csr &A0)
       lv.ut = dalloc_n<double>((size_t) n);
       lv.r = dalloc_n<double>((size_t) n);
       if (p.cycle_fp32) {
-         make_fp32_view(*lv.A, lv.A32);
+         // l1-Jacobi levels with a solve-phase copy read that copy's values
+         const bool copy_only = (lv.sten.nslices > 0 || lv.ell.nslices > 0) &&
+                                j < num_levels - 1 && p.relax_type[1] == 18 && p.relax_type[2] == 18;
+         make_fp32_view(*lv.A, lv.A32, !copy_only);
          if (j < num_levels - 1) {
             make_fp32_view(lv.P, lv.P32);
             make_fp32_view(lv.R, lv.R32);
@@ -315,13 +349,20 @@ void AMGSolver::setup(const Csr &A0)
          }
       }
    }
+   const bool late = ell_started == 0;
    for (int j = ell_started; j < num_levels; j++) { start_ell(j); }
+   if (late) { finish_sten(); }
    // the solve phase runs after the copies are filled
    main_after_side();
    for (int j = 0; j < num_levels; j++) {
       Level &lv = L[j];
       lv.Av = *lv.A;
       lv.Av.ell = nullptr;
+      lv.Av.sten = nullptr;
+      if (lv.sten.nslices > 0) {
+         lv.Av.sten = &lv.sten;
+         if (p.cycle_fp32) { lv.A32.sten = &lv.sten; }
+      }
       if (lv.ell.stored > 0) {
          lv.Av.ell = &lv.ell;
          if (p.cycle_fp32) { lv.A32.ell = &lv.ell; }
@@ -519,7 +560,7 @@ void AMGSolver::cycle32(const double *f, double *u)
 // src/parcsr_ls/par_amg_solve.c:22-424
 const Csr &AMGSolver::solve_view(const Csr &A) const
 {
-   if (setup_done && !L.empty() && L[0].A == &A && L[0].Av.ell) { return L[0].Av; }
+   if (setup_done && !L.empty() && L[0].A == &A && (L[0].Av.ell || L[0].Av.sten)) { return L[0].Av; }
    return A;
 }
 

@@ -157,6 +157,33 @@ struct Ell
    void      free_all();
 };
 
+// What the probe of a stencil operator finds: its offsets col - row (0 first,
+// then ascending; 0 past the D-th) and the value of one entry of each
+struct StenHead
+{
+   int    ok, D, wmax, raw;       // raw: slices whose values are kept in full
+   int    off[32];
+   double v[32];
+};
+
+// Stencil copy of an operator for the solve phase (hx_stencil.hip): one mask
+// word a row, slices of 64 rows with no values (all equal to the table's), an
+// 8-bit code an entry and a dictionary of at most 256 values, or full values.
+struct Sten
+{
+   StenHead  tab = {};
+   int       nslices = 0;         // 0: no copy
+   int      *st = nullptr;        // probe's words
+   StenHead *head = nullptr;
+   unsigned *mask = nullptr;      // bit k: the row has step k
+   int      *info = nullptr;      // per slice: mode | 4 if all rows have all steps | values << 8
+   unsigned *codes = nullptr;     // four codes a word, word w of 64 rows contiguous
+   double   *dict = nullptr;      // 256 values a slice
+   double   *raw = nullptr;       // step k of 64 rows contiguous (only when some slice needs it)
+   float    *raw32 = nullptr;
+   void      free_all();
+};
+
 struct Csr
 {
    int       nrows = 0, ncols = 0;
@@ -166,6 +193,7 @@ struct Csr
    float    *a32 = nullptr;
    // not owned: when set, SpMV and l1-Jacobi run on this copy (same results)
    const Ell *ell = nullptr;
+   const Sten *sten = nullptr;
    void      free_all();
    void      alloc(int n, int nc, long long nz, bool values = true);
 };
@@ -177,6 +205,21 @@ struct Csr
 // ell_fill launches the copy on s
 bool ell_plan(const Csr &A, Ell &E, double max_pad, int min_rows, bool fp32);
 void ell_fill(const Csr &A, Ell &E, bool fp32, hipStream_t s);
+
+// The stencil copy, in steps on stream s: sten_probe launches the search for
+// the offsets (false: not worth it for this operator), sten_take reads its
+// result once s has finished (false: no stencil), sten_fill builds the copy,
+// and sten_fill_raw, once s has finished and sten_raw_slices() says that some
+// slice needs it, the full values
+bool sten_probe(const Csr &A, Sten &S, int min_rows, hipStream_t s);
+bool sten_take(Sten &S);
+void sten_fill(const Csr &A, Sten &S, hipStream_t s);
+int  sten_raw_slices();
+void sten_fill_raw(const Csr &A, Sten &S, bool fp32, hipStream_t s);
+template <typename V, typename X, bool DOT>
+int sten_spmv(const Csr &A, X alpha, const X *x, X beta, const X *b, X *y, double *part);
+template <typename V, typename X>
+void sten_relax_l1(const Csr &A, const X *f, const X *u, const X *l1, X w, X *uo);
 
 void csr_copy(const Csr &src, Csr &dst);
 void csr_to_host(const Csr &A, std::vector<int> &ia, std::vector<int> &ja, std::vector<double> &a);

@@ -49,7 +49,8 @@ struct Level
    Csr     Arev;                // rows of A reversed, for backward hybrid Gauss-Seidel
    int     max_row = -1;        // longest row of A (hybrid Gauss-Seidel chunking)
    Ell     ell;                 // sliced-ELL copy of A for the solve phase (when built)
-   Csr     Av;                  // the operator as the solve phase sees it: *A plus ell
+   Sten    sten;                // stencil copy of A instead of ell (grid operators)
+   Csr     Av;                  // the operator as the solve phase sees it: *A plus ell or sten
 };
 
 struct AMGParams

@@ -575,6 +575,7 @@ void Csr::free_all()
    ia = ja = nullptr; a = nullptr; a32 = nullptr;
    nrows = ncols = 0; nnz = 0;
    ell = nullptr;
+   sten = nullptr;
 }
 
 void Ell::free_all()

@@ -707,6 +707,12 @@ static int launch_spmv(const Csr &A, const V *vals, X alpha, const X *x, X beta,
    double bytes = (double) A.nnz * (4.0 + vbytes) + 4.0 * (A.nrows + 1) +
                   (double) sizeof(X) * (A.ncols + A.nrows) + (beta != (X) 0 ? sizeof(X) * (double) A.nrows : 0.0) +
                   (ZR ? 2.0 * sizeof(X) * A.nrows : 0.0);
+   if constexpr (!ZR) {
+      if (A.sten) {
+         TimedLaunch tl(cls, bytes);
+         return sten_spmv<V, X, DOT>(A, alpha, x, beta, b, y, part);
+      }
+   }
    if (A.ell) {
       const Ell &E = *A.ell;
       const int nb = grid_for_groups(A.nrows, 64);
@@ -747,7 +753,7 @@ void spmv(const Csr &A, double alpha, const double *x, double beta, const double
 void spmv32(const Csr &A, float alpha, const float *x, float beta, const float *b, float *y,
             const char *cls)
 {
-   if (!A.a32) { fail(HYPRE_ERROR_GENERIC, "FP32 values missing"); }
+   if (!A.a32 && !A.ell && !A.sten) { fail(HYPRE_ERROR_GENERIC, "FP32 values missing"); }
    launch_spmv<float, float, false>(A, A.a32, alpha, x, beta, b, y, nullptr, cls, 4.0);
 }
 
@@ -852,6 +858,8 @@ static void launch_relax_l1(const Csr &A, const V *vals, const X *f, const X *u,
    if (zero) {
       const int nb = std::max(1, std::min((A.nrows + BS - 1) / BS, 16384));
       k_relax_l1_zero<X><<<nb, BS, 0, s>>>(A.nrows, f, l1, w, uo);
+   } else if (A.sten) {
+      sten_relax_l1<V, X>(A, f, u, l1, w, uo);
    } else if (A.ell) {
       const Ell &E = *A.ell;
       const int nb = grid_for_groups(A.nrows, 64);

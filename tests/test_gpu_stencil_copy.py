@@ -1,0 +1,127 @@
+"""The stencil copy of the fine operator gives the bits of the CSR kernels.
+
+solve_format 0 runs the CSR kernels, format 1 (default) the stencil copy where
+the fine operator's columns differ from the row by at most 32 offsets: slices
+of 128 rows with no values, with a dictionary of at most 256, or with full
+values.  A V-cycle in FP64 and FP32 must agree bit for bit between the two on
+grids whose slices are cut by lines, planes and the matrix's end, on the
+table sizes with an unrolled kernel (5, 7, 9, 19, 27) and others, at 32 and
+33 offsets, and on rows that are not sorted (both fall back).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False, special=None):
+    """Rows diagonal first, then ascending, from (dx, dy, dz) offsets in
+    symmetric pairs; values 'const', 'few' (64 distinct couplings) or 'all'
+    (every coupling its own); missing: share of the pairs left out."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    n = nx * ny * nz
+    iz, iy, ix = np.unravel_index(np.arange(n), (nz, ny, nx))
+    rows, cols, vals = [], [], []
+    for dx, dy, dz in offsets:
+        if (dz, dy, dx) <= (0, 0, 0):
+            continue
+        jx, jy, jz = ix + dx, iy + dy, iz + dz
+        ok = (jx >= 0) & (jx < nx) & (jy >= 0) & (jy < ny) & (jz >= 0) & (jz < nz)
+        ok &= rng.random(n) >= missing
+        i = np.nonzero(ok)[0]
+        j = i + (dz * ny + dy) * nx + dx
+        v = {"const": np.ones(len(i)), "few": 0.5 + rng.integers(0, 64, len(i)) / 64.0,
+             "all": 0.5 + rng.random(len(i))}[values]
+        rows += [i, j]
+        cols += [j, i]
+        vals += [-v, -v]
+    off = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))), shape=(n, n))
+    off.sort_indices()
+    diag = 1e-2 - np.asarray(off.sum(axis=1)).ravel()
+    if values == "const":
+        diag[:] = diag.max()
+    ia = np.zeros(n + 1, np.int32)
+    ia[1:] = np.cumsum(np.diff(off.indptr) + 1)
+    ja, a = np.empty(ia[-1], np.int32), np.empty(ia[-1])
+    first = ia[:-1]
+    ja[first], a[first] = np.arange(n), diag
+    rest = np.ones(ia[-1], bool)
+    rest[first] = False
+    ja[rest], a[rest] = off.indices, off.data
+    if shuffle:
+        for r in range(0, n, 7):
+            s, e = ia[r] + 1, ia[r + 1]
+            ja[s:e], a[s:e] = ja[s:e][::-1].copy(), a[s:e][::-1].copy()
+    return ia, ja, a
+
+
+def box(r=1):
+    return [(x, y, z) for z in range(-r, r + 1) for y in range(-r, r + 1) for x in range(-r, r + 1)]
+
+
+P5 = [(0, 0, 0), (1, 0, 0), (-1, 0, 0), (0, 1, 0), (0, -1, 0)]
+P7 = P5 + [(0, 0, 1), (0, 0, -1)]
+P9 = [o for o in box() if o[2] == 0]
+P19 = [o for o in box() if sum(map(abs, o)) <= 2]
+P31 = [(k, 0, 0) for k in range(-15, 16)]
+P33 = [(k, 0, 0) for k in range(-16, 17)]
+
+CASES = {
+    "27_const_ragged": (17, 19, 23, box(), "const", {}),
+    "27_few": (21, 16, 17, box(), "few", {}),
+    "27_all": (19, 17, 16, box(), "all", {}),
+    "27_all_missing": (19, 17, 16, box(), "all", {"missing": 0.2}),
+    "27_thin": (2, 61, 47, box(), "few", {}),        # offsets of lines and planes overlap
+    "19_few": (18, 15, 19, P19, "few", {}),
+    "19_const": (64, 8, 8, P19, "const", {}),
+    "9_all": (131, 67, 1, P9, "all", {}),
+    "9_const": (128, 33, 1, P9, "const", {}),
+    "7_few_missing": (33, 13, 14, P7, "few", {"missing": 0.1}),
+    "7_const": (4, 33, 34, P7, "const", {}),
+    "5_all": (67, 71, 1, P5, "all", {}),
+    "31_few": (4111, 1, 1, P31, "few", {}),
+    "31_all_missing": (5003, 1, 1, P31, "all", {"missing": 0.3}),
+    "33_all": (4999, 1, 1, P33, "all", {}),           # one offset too many
+    "27_unsorted": (17, 17, 17, box(), "few", {"shuffle": True}),
+}
+
+
+def cycle(hx, A, fmt, f, fp32):
+    amg = hx.BoomerAMG(max_iter=1, tol=0.0, fp32_cycle=1 if fp32 else 0, solve_format=fmt)
+    amg.setup(A)
+    u = amg.cycle_host(f)
+    amg.destroy()
+    return u
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_vcycle_bits_equal_the_csr_kernels(hx, oracle, name, fp32):
+    nx, ny, nz, offsets, values, more = CASES[name]
+    print("[gpu-stencil]", name, fp32, flush=True)
+    A = hx.ParCSRMatrix.from_csr(*grid_matrix(nx, ny, nz, offsets, values, **more))
+    n, _ = A.dims()
+    assert n >= 4096
+    f = 2 * oracle.rand_stream(7, n) - 1
+    u0, u1 = cycle(hx, A, 0, f, fp32), cycle(hx, A, 1, f, fp32)
+    assert np.isfinite(u0).all() and np.abs(u0).max() > 0
+    bad = np.nonzero(u0.view(np.int64) != u1.view(np.int64))[0]
+    assert bad.size == 0, f"{bad.size} entries differ, first at {bad[:5]}"
+
+
+def test_product_with_dot_matches_the_csr_kernels(hx, oracle):
+    """PCG's s = A p on the copy (with <s, p>): same iterations, same solution
+    up to the order of the dot product's partial sums."""
+    out = []
+    for fmt in (0, 1):
+        A = hx.ParCSRMatrix.from_csr(*grid_matrix(21, 16, 17, box(), "few"))
+        n, _ = A.dims()
+        b, x = hx.ParVector(n, 2 * oracle.rand_stream(3, n) - 1), hx.ParVector(n)
+        pcg = hx.PCG(hx.BoomerAMG(solve_format=fmt), tol=1e-8)
+        pcg.setup(A, b, x)
+        pcg.solve(A, b, x)
+        out.append((pcg.num_iterations(), np.array(pcg.history()), x.get()))
+    assert out[0][0] == out[1][0]
+    np.testing.assert_allclose(out[1][1], out[0][1], rtol=1e-9)
+    np.testing.assert_allclose(out[1][2], out[0][2], rtol=1e-8, atol=1e-12 * np.abs(out[0][2]).max())

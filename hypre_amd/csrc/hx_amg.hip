@@ -655,15 +655,6 @@ static const Csr &mat_of(HYPRE_ParCSRMatrix A)
    return A->A;
 }
 
-static double dev_scalar_read(const double *d, int k = 1, double *out = nullptr)
-{
-   double *h = static_cast<double *>(pinned_scratch(64));
-   HX_HIP(hipMemcpyAsync(h, d, sizeof(double) * k, hipMemcpyDeviceToHost, stream()));
-   sync();
-   if (out) { for (int i = 0; i < k; i++) { out[i] = h[i]; } }
-   return h[0];
-}
-
 // device scalars of the PCG iteration live at byte offset 512 of the status block
 static double *scal_dev(int k) { return reinterpret_cast<double *>(device_flags()) + 64 + k; }
 
@@ -1002,11 +993,27 @@ HYPRE_Int HYPRE_ParCSRPCGSetup(HYPRE_Solver solver, HYPRE_ParCSRMatrix A, HYPRE_
    });
 }
 
+// the library's own preconditioners do nothing that a caller could see
+static bool own_precond(const PCGSolver *s)
+{
+   return !s->precond || s->precond == HYPRE_BoomerAMGSolve || s->precond == HYPRE_ParCSRDiagScale;
+}
+
+// a BoomerAMG preconditioner whose one cycle from a zero guess writes every
+// entry and reads none
+static bool cycle_writes_all(const PCGSolver *s, int n)
+{
+   if (s->precond != HYPRE_BoomerAMGSolve || !s->precond_solver || s->precond_solver->kind != 1) { return false; }
+   const auto *g = static_cast<const AMGSolver *>(s->precond_solver);
+   return g->setup_done && g->L[0].A->nrows == n && g->prm.max_iter >= 1 && !(g->prm.tol > 0.) &&
+          g->prm.print_level <= 1 && g->prm.logging <= 1;
+}
+
 static void apply_precond(PCGSolver *s, HYPRE_ParCSRMatrix A, hypre_ParVector_struct *rhs,
                           hypre_ParVector_struct *out)
 {
    // ClearVector (par_krylov_func.c:260) then the preconditioner
-   fill(out->n, 0.0, out->d);
+   if (s->precond && !cycle_writes_all(s, out->n)) { fill(out->n, 0.0, out->d); }
    out->all_zeros = true;
    if (s->precond) {
       s->precond(s->precond_solver, A, rhs, out);
@@ -1089,8 +1096,7 @@ HYPRE_Int HYPRE_ParCSRPCGSolve(HYPRE_Solver solver, HYPRE_ParCSRMatrix A, HYPRE_
       int i = 0;
       const double REAL_MIN = 2.2250738585072014e-308;
       const double TRUE_MIN = 4.9406564584124654e-324;
-      double *d_sdotp = scal_dev(0), *d_alpha = scal_dev(1), *d_gam = scal_dev(2),
-             *d_beta = scal_dev(4), *d_gold = scal_dev(5);
+      double *d_sdotp = scal_dev(0);
       double gamma_old = 0.0;
       if (s->print_level > 1) {
          printf("<b,b>: %e\n\n Iters       ||r||_2     conv.rate  ||r||_2/||b||_2\n", bi_prod);
@@ -1099,9 +1105,21 @@ HYPRE_Int HYPRE_ParCSRPCGSolve(HYPRE_Solver solver, HYPRE_ParCSRMatrix A, HYPRE_
       double prev_norm = std::sqrt(i_prod_0);
       while ((i + 1) <= s->max_iter) {
          i++;
-         // s = A p, sdotp = <s,p>
-         spmv_dot(M, p->d, sv->d, d_sdotp, "spmv_A0");
-         double sdotp = dev_scalar_read(d_sdotp);
+         // s = A p, sdotp = <s,p>; x += alpha p ; r -= alpha s ; s = C r ;
+         // gamma = <r,s> ; i_prod = <r,r>.  sdotp comes with the last two: the
+         // device divides and, where the iteration breaks off at alpha, leaves
+         // x and r alone.  Only a caller's own preconditioner, which must not
+         // see such an iteration, has the host look first.
+         const DotParts sp = spmv_dot(M, p->d, sv->d, "spmv_A0");
+         double dots[3] = {0.0, 0.0, 0.0};
+         const bool ahead = own_precond(s);
+         if (!ahead) { dots[2] = dot_sum(sp); }
+         if (ahead || !pcg_alpha_stops(gamma, dots[2], s->skip_break)) {
+            pcg_update_xr(n, sp, gamma, s->skip_break, d_sdotp, p->d, sv->d, x->d, r->d);
+            apply_precond(s, A, r, sv);
+            dot2_sums(dot2_parts(n, r->d, sv->d), d_sdotp, dots);
+         }
+         const double sdotp = dots[2];
          if (sdotp == 0.0) {
             set_error(HYPRE_ERROR_CONV, "Zero sdotp value in PCG");
             if (i == 1) { i_prod = i_prod_0; }
@@ -1118,20 +1136,10 @@ HYPRE_Int HYPRE_ParCSRPCGSolve(HYPRE_Solver solver, HYPRE_ParCSRMatrix A, HYPRE_
             set_error(HYPRE_ERROR_CONV, "Subnormal alpha value in PCG");
             if (s->skip_break < 1) { if (i == 1) { i_prod = i_prod_0; } break; }
          }
-         gamma_old = gamma;
-         // x += alpha p ; r -= alpha s
-         double *ha = static_cast<double *>(pinned_scratch(64));
-         ha[0] = alpha;
-         HX_HIP(hipMemcpyAsync(d_alpha, ha, sizeof(double), hipMemcpyHostToDevice, stream()));
-         pcg_update_xr(n, d_alpha, p->d, sv->d, x->d, r->d);
          x->all_zeros = false;
-         // s = C r ; gamma = <r,s> ; i_prod = <r,r>
-         apply_precond(s, A, r, sv);
-         dot2_dev(n, r->d, sv->d, d_gam);
-         double g2[2];
-         dev_scalar_read(d_gam, 2, g2);
-         gamma = g2[0];
-         i_prod = s->two_norm ? g2[1] : gamma;
+         gamma_old = gamma;
+         gamma = dots[0];
+         i_prod = s->two_norm ? dots[1] : gamma;
          double nrm = std::sqrt(i_prod);
          s->history.push_back(bi_prod > 0.0 ? std::sqrt(i_prod / bi_prod) : 0.0);
          if (s->print_level > 1) {
@@ -1172,13 +1180,9 @@ HYPRE_Int HYPRE_ParCSRPCGSolve(HYPRE_Solver solver, HYPRE_ParCSRMatrix A, HYPRE_
             if (s->skip_break < 1) { if (i == 1) { i_prod = i_prod_0; } break; }
          }
          // beta = gamma / gamma_old ; p = s + beta p
-         double beta = gamma / gamma_old;
-         double *hb = static_cast<double *>(pinned_scratch(64));
-         hb[1] = beta;
-         HX_HIP(hipMemcpyAsync(d_beta, hb + 1, sizeof(double), hipMemcpyHostToDevice, stream()));
-         pcg_update_p(n, d_beta, sv->d, p->d);
+         const double beta = gamma / gamma_old;
+         pcg_update_p(n, beta, sv->d, p->d);
       }
-      (void) d_gold;
       if (i >= s->max_iter && (i_prod / bi_prod) >= eps && eps > 0) {
          set_error(HYPRE_ERROR_CONV, "Reached max iterations in PCG before convergence");
       }

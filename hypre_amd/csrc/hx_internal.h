@@ -236,8 +236,17 @@ void spmv_zero_relax(const Csr &A, const double *x, double *y, const double *l1,
                      double *u, const char *cls);
 void spmv32_zero_relax(const Csr &A, const float *x, float *y, const float *l1, float w, float *u,
                        const char *cls);
-// s = A p and part[] = per-block partial sums of s.*p (deterministic)
-void spmv_dot(const Csr &A, const double *p, double *s, double *dot_out_dev, const char *cls);
+// the n partial sums of a dot product, one a block (deterministic)
+struct DotParts
+{
+   const double *part;
+   int           n;
+};
+constexpr int DOT_STRIDE = 8192;   // most blocks that form partial sums
+double  *dot_parts();              // two sets of them, DOT_STRIDE apart
+// s = A p and the partial sums of <s, p>; their sum (waits)
+DotParts spmv_dot(const Csr &A, const double *p, double *s, const char *cls);
+double   dot_sum(const DotParts &d);
 // l1-Jacobi: u_out = u + (w*f - w*A*u)./l1 ; zero_guess: u_out = (w*f)./l1
 void relax_l1(const Csr &A, const double *f, const double *u, const double *l1, double w,
               double *u_out, bool zero_guess, const char *cls);
@@ -265,19 +274,33 @@ void relax_hgs_32(int type, const Csr &A, const Csr *Arev, int max_row, const fl
                   bool zero_guess, const char *cls);
 // BLAS-1
 double dot(int n, const double *x, const double *y);
-void   dot_dev(int n, const double *x, const double *y, double *out_dev);
-void   dot2_dev(int n, const double *r, const double *s, double *out2_dev); // <r,s>, <r,r>
+// partial sums of <r,s> and <r,r> (dot_parts), and, waiting for them, the two
+// sums and the device value *more_dev
+int    dot2_parts(int n, const double *r, const double *s);
+void   dot2_sums(int nb, const double *more_dev, double *out3);
 void   axpy(int n, double alpha, const double *x, double *y);               // y += alpha x
 void   scale(int n, double alpha, double *x);
 void   fill(int n, double v, double *x);
 void   fill32(int n, float v, float *x);
 void   copy(int n, const double *x, double *y);
-void   pcg_update_xr(int n, const double *alpha_dev, const double *p, const double *s, double *x,
-                     double *r);                                            // x += a p; r -= a s
-void   pcg_update_p(int n, const double *beta_dev, const double *s, double *p); // p = beta p + s
+// whether pcg.c leaves the iteration before its updates: <s,p> zero, or alpha
+// not positive, below the least number or subnormal and not skipped
+__host__ __device__ inline bool pcg_alpha_stops(double gamma, double sdotp, int skip_break)
+{
+   if (sdotp == 0.0) { return true; }
+   const double alpha = gamma / sdotp;
+   if (alpha <= 0.0) { return skip_break < 3; }
+   if (!(alpha >= 4.9406564584124654e-324)) { return skip_break < 2; }
+   if (!(alpha >= 2.2250738585072014e-308)) { return skip_break < 1; }
+   return false;
+}
+// alpha = gamma / <s,p>; x += alpha p; r -= alpha s (nothing where
+// pcg_alpha_stops); <s,p> to *sdotp_dev
+void   pcg_update_xr(int n, const DotParts &sp, double gamma, int skip_break, double *sdotp_dev,
+                     const double *p, const double *s, double *x, double *r);
+void   pcg_update_p(int n, double beta, const double *s, double *p);        // p = beta p + s
 void   d2f(int n, const double *x, float *y);
 void   f2d(int n, const float *x, double *y);
-void   scalar_div(const double *num, const double *den, double *out);       // device scalars
 // coarsest dense solve, column-major matrix (relax type 9)
 void   gselim_solve(int n, const double *Amat_dev, const double *f, double *u);
 void   gselim_solve32(int n, const double *Amat_dev, const float *f, float *u);

@@ -283,10 +283,10 @@ __global__ __launch_bounds__(BS) void k_spmv_w(int n, const int *__restrict__ ia
    }
 }
 
-__global__ __launch_bounds__(BS) void k_reduce_parts(const double *__restrict__ part, int np,
-                                                     double *__restrict__ out)
+// the sum of np partial sums, in every thread of the block, always in the same
+// order
+__device__ __forceinline__ double block_sum_parts(const double *__restrict__ part, int np, double *sh)
 {
-   __shared__ double sh[BS];
    double s = 0.0;
    for (int i = threadIdx.x; i < np; i += BS) { s += part[i]; }
    sh[threadIdx.x] = s;
@@ -295,15 +295,43 @@ __global__ __launch_bounds__(BS) void k_reduce_parts(const double *__restrict__ 
       if (threadIdx.x < off) { sh[threadIdx.x] += sh[threadIdx.x + off]; }
       __syncthreads();
    }
-   if (threadIdx.x == 0) { *out = sh[0]; }
+   const double sum = sh[0];
+   __syncthreads();
+   return sum;
 }
 
+__global__ __launch_bounds__(BS) void k_reduce_parts(const double *__restrict__ part, int np,
+                                                     double *__restrict__ out)
+{
+   __shared__ double sh[BS];
+   const double s = block_sum_parts(part, np, sh);
+   if (threadIdx.x == 0) { *out = s; }
+}
+
+// two sums side by side and a third value beside them: out[0..2]
+__global__ __launch_bounds__(BS) void k_reduce_parts2(const double *__restrict__ part, int np,
+                                                      const double *__restrict__ more,
+                                                      double *__restrict__ out)
+{
+   __shared__ double sh[BS];
+   const double a = block_sum_parts(part, np, sh);
+   const double b = block_sum_parts(part + DOT_STRIDE, np, sh);
+   if (threadIdx.x == 0) {
+      out[0] = a;
+      out[1] = b;
+      out[2] = *more;
+   }
+}
+
+// partial sums of a launch's blocks: two sets of at most DOT_STRIDE, then the
+// set of the product <s, p>, which is still read while the next two are formed
 static double *g_part = nullptr;
 static double *parts()
 {
-   if (!g_part) { g_part = dalloc_n<double>(8192 * 2); }
+   if (!g_part) { g_part = dalloc_n<double>(DOT_STRIDE * 3); }
    return g_part;
 }
+double *dot_parts() { return parts(); }
 
 static int grid_for_groups(int n, int rw)
 {
@@ -772,11 +800,20 @@ void spmv32_zero_relax(const Csr &A, const float *x, float *y, const float *l1, 
                                           w, u);
 }
 
-void spmv_dot(const Csr &A, const double *p, double *s, double *dot_out_dev, const char *cls)
+DotParts spmv_dot(const Csr &A, const double *p, double *s, const char *cls)
 {
-   const int nb = launch_spmv<double, double, true>(A, A.a, 1.0, p, 0.0, nullptr, s, parts(), cls, 8.0);
-   k_reduce_parts<<<1, BS, 0, stream()>>>(parts(), std::max(nb, 0), dot_out_dev);
+   double *part = parts() + 2 * DOT_STRIDE;
+   const int nb = launch_spmv<double, double, true>(A, A.a, 1.0, p, 0.0, nullptr, s, part, cls, 8.0);
+   return DotParts{part, std::max(nb, 0)};
+}
+
+double dot_sum(const DotParts &d)
+{
+   double *h = static_cast<double *>(pinned_scratch(64));
+   k_reduce_parts<<<1, BS, 0, stream()>>>(d.part, d.n, h);
    HX_LAUNCH_CHECK();
+   sync();
+   return h[0];
 }
 
 // ---------------------------------------------------------------- relaxation
@@ -1449,35 +1486,37 @@ __global__ __launch_bounds__(BS) void k_dot2_part(int n, const double *__restric
    }
    if (threadIdx.x == 0) {
       part[blockIdx.x] = sh[0][0];
-      part[8192 + blockIdx.x] = sh[1][0];
+      part[DOT_STRIDE + blockIdx.x] = sh[1][0];
    }
 }
 
-void dot_dev(int n, const double *x, const double *y, double *out_dev)
-{
-   int nb = blas_grid(n);
-   TimedLaunch tl("blas", 16.0 * n);
-   k_dot_part<<<nb, BS, 0, stream()>>>(n, x, y, parts());
-   k_reduce_parts<<<1, BS, 0, stream()>>>(parts(), nb, out_dev);
-   HX_LAUNCH_CHECK();
-}
-
-void dot2_dev(int n, const double *r, const double *s, double *out2_dev)
+int dot2_parts(int n, const double *r, const double *s)
 {
    int nb = blas_grid(n);
    TimedLaunch tl("blas", 16.0 * n);
    k_dot2_part<<<nb, BS, 0, stream()>>>(n, r, s, parts());
-   k_reduce_parts<<<1, BS, 0, stream()>>>(parts(), nb, out2_dev);
-   k_reduce_parts<<<1, BS, 0, stream()>>>(parts() + 8192, nb, out2_dev + 1);
    HX_LAUNCH_CHECK();
+   return nb;
 }
 
+void dot2_sums(int nb, const double *more_dev, double *out3)
+{
+   double *h = static_cast<double *>(pinned_scratch(64));
+   k_reduce_parts2<<<1, BS, 0, stream()>>>(parts(), nb, more_dev, h);
+   HX_LAUNCH_CHECK();
+   sync();
+   for (int k = 0; k < 3; k++) { out3[k] = h[k]; }
+}
+
+// the last reduction writes its sum to pinned host memory: no copy of its own
 double dot(int n, const double *x, const double *y)
 {
-   double *d = reinterpret_cast<double *>(device_flags() + 32);
-   dot_dev(n, x, y, d);
+   int nb = blas_grid(n);
    double *h = static_cast<double *>(pinned_scratch(64));
-   HX_HIP(hipMemcpyAsync(h, d, sizeof(double), hipMemcpyDeviceToHost, stream()));
+   TimedLaunch tl("blas", 16.0 * n);
+   k_dot_part<<<nb, BS, 0, stream()>>>(n, x, y, parts());
+   k_reduce_parts<<<1, BS, 0, stream()>>>(parts(), nb, h);
+   HX_LAUNCH_CHECK();
    sync();
    return h[0];
 }
@@ -1507,22 +1546,31 @@ __global__ void k_copy(int n, const double *__restrict__ x, double *__restrict__
       y[i] = x[i];
    }
 }
-// x += alpha p ; r += (-alpha) s   (two hypre_ParKrylovAxpy calls, pcg.c)
-__global__ void k_pcg_xr(int n, const double *__restrict__ ad, const double *__restrict__ p,
-                         const double *__restrict__ s, double *__restrict__ x,
-                         double *__restrict__ r)
+// alpha = gamma / <s, p>, then x += alpha p ; r += (-alpha) s (pcg.c; two
+// hypre_ParKrylovAxpy calls).  Every block sums <s, p>'s partial sums by
+// itself, so the step needs neither a reduction nor the host in between; a
+// step that pcg.c would break off before the updates leaves x and r alone, and
+// the host sees why from <s, p>, kept in *sdotp.
+__global__ __launch_bounds__(BS) void k_pcg_xr(int n, const double *__restrict__ part, int np,
+                                               double gamma, int skip_break,
+                                               double *__restrict__ sdotp,
+                                               const double *__restrict__ p,
+                                               const double *__restrict__ s, double *__restrict__ x,
+                                               double *__restrict__ r)
 {
-   double alpha = *ad, malpha = -alpha;
+   __shared__ double sh[BS];
+   const double sp = block_sum_parts(part, np, sh);
+   if (blockIdx.x == 0 && threadIdx.x == 0) { *sdotp = sp; }
+   if (pcg_alpha_stops(gamma, sp, skip_break)) { return; }
+   const double alpha = gamma / sp, malpha = -alpha;
    for (long long i = (long long) blockIdx.x * BS + threadIdx.x; i < n; i += (long long) gridDim.x * BS) {
       x[i] += alpha * p[i];
       r[i] += malpha * s[i];
    }
 }
 // p = beta p ; p += 1.0 s   (ScaleVector + Axpy, pcg.c)
-__global__ void k_pcg_p(int n, const double *__restrict__ bd, const double *__restrict__ s,
-                        double *__restrict__ p)
+__global__ void k_pcg_p(int n, double beta, const double *__restrict__ s, double *__restrict__ p)
 {
-   double beta = *bd;
    for (long long i = (long long) blockIdx.x * BS + threadIdx.x; i < n; i += (long long) gridDim.x * BS) {
       double t = beta * p[i];
       p[i] = t + s[i];
@@ -1540,7 +1588,6 @@ __global__ void k_f2d(int n, const float *__restrict__ x, double *__restrict__ y
       y[i] = (double) x[i];
    }
 }
-__global__ void k_sdiv(const double *num, const double *den, double *out) { *out = *num / *den; }
 
 void axpy(int n, double alpha, const double *x, double *y)
 {
@@ -1572,17 +1619,23 @@ void copy(int n, const double *x, double *y)
    k_copy<<<blas_grid(n), BS, 0, stream()>>>(n, x, y);
    HX_LAUNCH_CHECK();
 }
-void pcg_update_xr(int n, const double *alpha_dev, const double *p, const double *s, double *x,
-                   double *r)
+void pcg_update_xr(int n, const DotParts &d, double gamma, int skip_break, double *sdotp_dev,
+                   const double *p, const double *s, double *x, double *r)
 {
    TimedLaunch tl("blas", 40.0 * n);
-   k_pcg_xr<<<blas_grid(n), BS, 0, stream()>>>(n, alpha_dev, p, s, x, r);
+   DotParts q = d;
+   if (d.n > 2048) {
+      // too many for every block to sum again: once, beforehand
+      k_reduce_parts<<<1, BS, 0, stream()>>>(d.part, d.n, parts());
+      q = DotParts{parts(), 1};
+   }
+   k_pcg_xr<<<blas_grid(n), BS, 0, stream()>>>(n, q.part, q.n, gamma, skip_break, sdotp_dev, p, s, x, r);
    HX_LAUNCH_CHECK();
 }
-void pcg_update_p(int n, const double *beta_dev, const double *s, double *p)
+void pcg_update_p(int n, double beta, const double *s, double *p)
 {
    TimedLaunch tl("blas", 24.0 * n);
-   k_pcg_p<<<blas_grid(n), BS, 0, stream()>>>(n, beta_dev, s, p);
+   k_pcg_p<<<blas_grid(n), BS, 0, stream()>>>(n, beta, s, p);
    HX_LAUNCH_CHECK();
 }
 void d2f(int n, const double *x, float *y)
@@ -1597,12 +1650,6 @@ void f2d(int n, const float *x, double *y)
    k_f2d<<<blas_grid(n), BS, 0, stream()>>>(n, x, y);
    HX_LAUNCH_CHECK();
 }
-void scalar_div(const double *num, const double *den, double *out)
-{
-   k_sdiv<<<1, 1, 0, stream()>>>(num, den, out);
-   HX_LAUNCH_CHECK();
-}
-
 // ---------------------------------------------------------------- coarsest solve
 // hypre_gselim (src/utilities/gselim.h) on the column-major matrix of
 // par_gauss_elim.c:312-316, one block: the updates of one elimination step

@@ -70,13 +70,19 @@ __device__ __forceinline__ X row_dot(int s, int e, int lane, const int *__restri
 constexpr int SW = 512;          // default window (entries); 1024 selectable
 constexpr int WPB = BS / 64;   // waves per block
 
-// rows per block: one row per lane, fewer only for very long rows so that a
-// lane's serial sum stays short
+// rows per block: one row per lane; fewer for very long rows, so that a lane's
+// serial sum stays short, and on small matrices, where the round trips of one
+// wave are the whole time: down to about 128 entries a block while there are
+// not yet 4096 blocks (half the waves the device holds).  Measured on whole
+// solves, without -> with: one V-cycle on an irregular matrix of 336,000 rows
+// 313 -> 278 us, PCG on 7-point 30^3 1.89 -> 1.64 ms, 117x131x109 6.72 -> 6.18
+// ms, 256^3 57.2 -> 56.3 ms.
 static int pick_rw(long long nnz, int n)
 {
    double avg = n > 0 ? (double) nnz / n : 1.0;
    int rw = 64;
    while (rw > 1 && rw * avg > 4 * SW) { rw >>= 1; }
+   while (rw > 4 && rw * avg > 128.0 && (n + rw - 1) / rw < 4096) { rw >>= 1; }
    return rw;
 }
 
@@ -85,15 +91,16 @@ __device__ __forceinline__ void wave_fence() { __builtin_amdgcn_wave_barrier(); 
 // window size of the SpMV / l1-Jacobi kernels: 1024 entries (measured faster
 // on the 27-point 200^3 fine level than 512), or 512 when the environment sets
 // HYPRE_MI355X_SPMV_WINDOW=512 (read once); 256 or 512 for matrices whose
-// 64-row groups hold at most that many entries on average (interpolation,
-// 7-point operators), where a wide window would mostly issue masked loads
-static int spmv_window(long long nnz, int n)
+// blocks of rw rows hold at most that many entries on average (interpolation,
+// 7-point operators, small levels), where a wide window would mostly issue
+// masked loads
+static int spmv_window(long long nnz, int n, int rw)
 {
    static int w = [] {
       const char *e = std::getenv("HYPRE_MI355X_SPMV_WINDOW");
       return (e && std::atoi(e) == SW) ? SW : 1024;
    }();
-   const double group = n > 0 ? (double) nnz / n * 64.0 : 0.0;
+   const double group = n > 0 ? (double) nnz / n * rw : 0.0;
    if (group <= 256.0) { return 256; }
    if (group <= 512.0) { return 512; }
    return w;
@@ -755,7 +762,7 @@ static int launch_spmv(const Csr &A, const V *vals, X alpha, const X *x, X beta,
    const int nb = grid_for_groups(A.nrows, rw);
    TimedLaunch tl(cls, bytes);
    hipStream_t s = stream();
-   const int sw = spmv_window(A.nnz, A.nrows);
+   const int sw = spmv_window(A.nnz, A.nrows, rw);
    dispatch_rw(rw, [&](auto c) {
       if (sw == 1024) {
          k_spmv_w<decltype(c)::value, 1024, V, X, DOT, ZR><<<nb, BS, 0, s>>>(
@@ -905,7 +912,7 @@ static void launch_relax_l1(const Csr &A, const V *vals, const X *f, const X *u,
    } else {
       const int rw = pick_rw(A.nnz, A.nrows);
       const int nb = grid_for_groups(A.nrows, rw);
-      const int sw = spmv_window(A.nnz, A.nrows);
+      const int sw = spmv_window(A.nnz, A.nrows, rw);
       dispatch_rw(rw, [&](auto c) {
          if (sw == 1024) {
             k_relax_l1_w<decltype(c)::value, 1024, V, X><<<nb, BS, 0, s>>>(A.nrows, A.ia, A.ja, vals,

@@ -110,6 +110,13 @@ typedef int hx_int2 __attribute__((ext_vector_type(2)));
 typedef double hx_dbl2 __attribute__((ext_vector_type(2)));
 typedef float hx_flt2 __attribute__((ext_vector_type(2)));
 
+// a row's operands of an epilogue
+template <typename X>
+struct RowOps
+{
+   X a, b, c;
+};
+
 // entries p and p+1 (p even) of the column indices and values
 template <typename V>
 __device__ __forceinline__ void load_pair(const int *__restrict__ ja, const V *__restrict__ a, int p,
@@ -129,26 +136,30 @@ __device__ __forceinline__ void load_pair(const int *__restrict__ ja, const V *_
    }
 }
 
-// Rows [R0, R1) of A times x; epi(row, t) is called once per row, by the lane
-// that owns it, with t the row's sum.  The matrix is streamed once: its loads
+// Rows [R0, R1) of A times x; epi(row, t, ops) is called once per row, by the
+// lane that owns it, with t the row's sum and ops = pre(row), the row's other
+// operands, loaded together with its bounds: asked for after the sum they cost
+// one more round trip, a tenth of a small level's kernel.  The matrix is streamed once: its loads
 // are non-temporal so that x stays in L2, and the next window's loads are
 // issued before the current window's products are summed.  Windows start at
 // the even entry at or below the range's first entry; pair loads past the
 // range read the last pair inside it (every CSR array is allocated with at
 // least one element of slack) and are masked when used.
-template <int RW, int SW, typename V, typename X, class Epi>
+template <int RW, int SW, typename V, typename X, class Pre, class Epi>
 __device__ __forceinline__ void rows_stream(int R0, int R1, int lane, const int *__restrict__ ia,
                                             const int *__restrict__ ja, const V *__restrict__ a,
-                                            const X *__restrict__ x, X *sbuf, Epi epi)
+                                            const X *__restrict__ x, X *sbuf, Pre pre, Epi epi)
 {
    constexpr int G = SW / 128;
    if (R0 >= R1) { return; }
    int rb = R0;
    int nr = min(RW, R1 - rb);
    int rs = 0, re = 0;
+   decltype(pre(0)) po = {}, po2 = {};
    if (lane < nr) {
       rs = ia[rb + lane];
       re = ia[rb + lane + 1];
+      po = pre(rb + lane);
    }
    // bounds of the next block, loaded one block ahead
    int nr2 = min(RW, R1 - (rb + RW));
@@ -156,6 +167,7 @@ __device__ __forceinline__ void rows_stream(int R0, int R1, int lane, const int 
    if (lane < nr2) {
       rs2 = ia[rb + RW + lane];
       re2 = ia[rb + RW + lane + 1];
+      po2 = pre(rb + RW + lane);
    }
    const int base = __shfl(rs, 0, 64);
    const int end = ia[R1];
@@ -164,7 +176,7 @@ __device__ __forceinline__ void rows_stream(int R0, int R1, int lane, const int 
    if (base >= end) {
       // no entries: every row sums to zero
       while (nr > 0) {
-         if (lane < nr) { epi(rb + lane, t); }
+         if (lane < nr) { epi(rb + lane, t, pre(rb + lane)); }
          rb += RW;
          nr = min(RW, R1 - rb);
       }
@@ -224,18 +236,20 @@ __device__ __forceinline__ void rows_stream(int R0, int R1, int lane, const int 
          }
          if (bend > we) { break; }
          // the block's rows end in this window
-         if (lane < nr) { epi(rb + lane, t); }
+         if (lane < nr) { epi(rb + lane, t, po); }
          t = 0;
          rb += RW;
          nr = nr2;
          rs = rs2;
          re = re2;
+         po = po2;
          if (nr <= 0) { break; }
          bend = __shfl(re, nr - 1, 64);
          nr2 = min(RW, R1 - (rb + RW));
          if (lane < nr2) {
             rs2 = ia[rb + RW + lane];
             re2 = ia[rb + RW + lane + 1];
+            po2 = pre(rb + RW + lane);
          }
       }
       wave_fence();
@@ -272,12 +286,21 @@ __global__ __launch_bounds__(BS) void k_spmv_w(int n, const int *__restrict__ ia
    int R0, R1;
    wave_rows<RW>(n, blk, wv, nb, R0, R1);
    double acc = 0.0;
-   rows_stream<RW, SW, V, X>(R0, R1, lane, ia, ja, a, x, sbuf, [&](int row, X t) {
-      const X v = (beta == (X) 0) ? alpha * t : alpha * t + beta * b[row];
-      y[row] = v;
-      if (DOT) { acc += (double) v * (double) x[row]; }
-      if (ZR) { zu[row] = (X) 0 + (zw * v) / zl1[row]; }
-   });
+   rows_stream<RW, SW, V, X>(
+      R0, R1, lane, ia, ja, a, x, sbuf,
+      [&](int row) {
+         RowOps<X> o{(X) 0, (X) 0, (X) 0};
+         if (beta != (X) 0) { o.a = b[row]; }
+         if (DOT) { o.b = x[row]; }
+         if (ZR) { o.c = zl1[row]; }
+         return o;
+      },
+      [&](int row, X t, const RowOps<X> &o) {
+         const X v = (beta == (X) 0) ? alpha * t : alpha * t + beta * o.a;
+         y[row] = v;
+         if (DOT) { acc += (double) v * (double) o.b; }
+         if (ZR) { zu[row] = (X) 0 + (zw * v) / o.c; }
+      });
    if (DOT) {
       __shared__ double sh[BS];
       sh[threadIdx.x] = acc;
@@ -440,12 +463,6 @@ __device__ __forceinline__ void ell_slice(int sl, int lane, int n, const int *__
    }
    if (r < n) { epi(r, t, pv); }
 }
-
-template <typename X>
-struct RowOps
-{
-   X a, b, c;
-};
 
 // slices of wave wv of block blk: a contiguous range, ranges in block order
 __device__ __forceinline__ void wave_slices(int ns, int blk, int wv, int nb, int &S0, int &S1)
@@ -873,10 +890,13 @@ __global__ __launch_bounds__(BS) void k_relax_l1_w(int n, const int *__restrict_
    X *sbuf = sbuf_all + wv * SW;
    int R0, R1;
    wave_rows<RW>(n, blk, wv, nb, R0, R1);
-   rows_stream<RW, SW, V, X>(R0, R1, lane, ia, ja, a, u, sbuf, [&](int row, X t) {
-      const X v = w * f[row] - w * t;
-      uo[row] = u[row] + v / l1[row];
-   });
+   rows_stream<RW, SW, V, X>(
+      R0, R1, lane, ia, ja, a, u, sbuf,
+      [&](int row) { return RowOps<X>{f[row], u[row], l1[row]}; },
+      [&](int row, X t, const RowOps<X> &o) {
+         const X v = w * o.a - w * t;
+         uo[row] = o.b + v / o.c;
+      });
 }
 
 // zero initial guess: u_out = (0 + w f) / l1, one thread per row

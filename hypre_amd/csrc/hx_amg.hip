@@ -279,6 +279,9 @@ void AMGSolver::setup(const Csr &A0)
    // option 4 for the l1 hybrid Gauss-Seidel types (par_amg_setup.c:3297-3317),
    // option 1 for l1-Jacobi, evaluated after it there and so taking precedence
    auto l1_gs = [](int t) { return t == 8 || t == 13 || t == 14; };
+   // the strength passes' flags of all levels in one read
+   std::vector<int> zero_l1(256, 0);
+   d2h(zero_l1.data(), l1_zero_flag(0), sizeof(int) * (size_t) std::min(num_levels, 256));
    for (int j = 0; j < num_levels; j++) {
       Range lrange("AMG Level-%d", j);    // par_amg_setup.c:3293-3297
       Range rrange("Relaxation-%d", j);
@@ -294,9 +297,7 @@ void AMGSolver::setup(const Csr &A0)
       }
       if (opt == 1 && lv.l1) {
          // computed with the level's strength matrix
-         int h = 0;
-         d2h(&h, l1_zero_flag(j), sizeof(int));
-         if (h) { g_error_arg = 1; set_error(HYPRE_ERROR_ARG, "zero l1 norm"); }
+         if (zero_l1[(size_t) std::min(j, 255)]) { g_error_arg = 1; set_error(HYPRE_ERROR_ARG, "zero l1 norm"); }
       } else if (opt == 1) {
          lv.l1 = dalloc_n<double>((size_t) n);
          l1_norms(*lv.A, lv.l1);

@@ -398,17 +398,67 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_apply(const int *in, int n, in
    }
 }
 
-// the three passes on the library stream; the total's 32-bit overflow flag,
-// the largest input and the 64-bit total land at flags + 8, 9 and 10..11
-static void scan_launch(const int *in, int *out, int n)
+// up to 16384 items by one block in one pass: 16 consecutive items a thread.
+// The three passes below take three launches, about 10 us whatever n; the
+// small levels of a setup scan some twenty such arrays.
+constexpr int SCAN_SMALL_BS = 1024, SCAN_SMALL_IT = 16, SCAN_SMALL = SCAN_SMALL_BS * SCAN_SMALL_IT;
+
+__global__ __launch_bounds__(SCAN_SMALL_BS) void k_scan_small(const int *in, int n, int *out, int *res)
 {
+   __shared__ long long wsum[SCAN_SMALL_BS / 64];
+   __shared__ int wmax[SCAN_SMALL_BS / 64];
+   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+   const int base = threadIdx.x * SCAN_SMALL_IT;
+   int v[SCAN_SMALL_IT];
+   long long s = 0;
+   int m = INT_MIN;
+#pragma unroll
+   for (int k = 0; k < SCAN_SMALL_IT; k++) {
+      v[k] = (base + k < n) ? in[base + k] : 0;
+      s += v[k];
+      if (base + k < n) { m = max(m, v[k]); }
+   }
+   long long incl = s;
+   for (int d = 1; d < 64; d <<= 1) {
+      const long long t = __shfl_up(incl, d, 64);
+      if (lane >= d) { incl += t; }
+      m = max(m, __shfl_xor(m, d, 64));
+   }
+   if (lane == 63) { wsum[wv] = incl; }
+   if (lane == 0) { wmax[wv] = m; }
+   __syncthreads();
+   long long run = incl - s;
+   for (int w = 0; w < wv; w++) { run += wsum[w]; }
+#pragma unroll
+   for (int k = 0; k < SCAN_SMALL_IT; k++) {
+      if (base + k < n) { out[base + k] = (int) run; }
+      run += v[k];
+   }
+   if (threadIdx.x == SCAN_SMALL_BS - 1) {
+      out[n] = (run > 0x7fffffffLL) ? 0x7fffffff : (int) run;
+      res[0] = (run > 0x7fffffffLL) ? 1 : 0;
+      int bm = wmax[0];
+      for (int w = 1; w < SCAN_SMALL_BS / 64; w++) { bm = max(bm, wmax[w]); }
+      res[1] = bm;
+      reinterpret_cast<long long *>(res + 2)[0] = run;
+   }
+}
+
+// the scan on the library stream; the total's 32-bit overflow flag, the
+// largest input and the 64-bit total go to res[0], res[1] and res[2..3]
+static void scan_launch(const int *in, int *out, int n, int *res)
+{
+   if (n <= SCAN_SMALL) {
+      k_scan_small<<<1, SCAN_SMALL_BS, 0, stream()>>>(in, n, out, res);
+      HX_LAUNCH_CHECK();
+      return;
+   }
    int ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
    long long *tiles = dalloc_n<long long>(ntiles);
    int *tmax = dalloc_n<int>(ntiles);
-   int *flags = device_flags();
    k_scan_tiles<<<ntiles, SCAN_BS, 0, stream()>>>(in, n, tiles, tmax);
    HX_LAUNCH_CHECK();
-   k_scan_sums<<<1, SCAN_BS, 0, stream()>>>(tiles, tmax, ntiles, out + n, flags + 8);
+   k_scan_sums<<<1, SCAN_BS, 0, stream()>>>(tiles, tmax, ntiles, out + n, res);
    HX_LAUNCH_CHECK();
    k_scan_apply<<<ntiles, SCAN_BS, 0, stream()>>>(in, n, out, tiles);
    HX_LAUNCH_CHECK();
@@ -417,6 +467,7 @@ static void scan_launch(const int *in, int *out, int n)
    dfree(tmax);
 }
 
+// the total comes back in pinned memory that the scan itself writes
 long long exclusive_scan(const int *in, int *out, int n, int *max_in)
 {
    if (n <= 0) {
@@ -425,9 +476,8 @@ long long exclusive_scan(const int *in, int *out, int n, int *max_in)
       if (max_in) { *max_in = 0; }
       return 0;
    }
-   scan_launch(in, out, n);
    int *h = static_cast<int *>(pinned_scratch(64));
-   HX_HIP(hipMemcpyAsync(h, device_flags() + 8, 4 * sizeof(int), hipMemcpyDeviceToHost, stream()));
+   scan_launch(in, out, n, h);
    sync();
    long long tot;
    std::memcpy(&tot, h + 2, sizeof(long long));
@@ -442,7 +492,7 @@ void exclusive_scan_nowait(const int *in, int *out, int n)
       dzero(out, sizeof(int));
       return;
    }
-   scan_launch(in, out, n);
+   scan_launch(in, out, n, device_flags() + 8);
 }
 
 __global__ void k_reduce_int(const int *__restrict__ in, int n, unsigned long long *sum, int *mx)

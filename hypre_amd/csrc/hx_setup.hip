@@ -134,12 +134,15 @@ struct RowClaim
    }
 };
 
+// eight claim counters and, between them, the pass's defer counter, cleared
+// together
 static int *claim_counters()
 {
    int *c = device_flags() + 512;
    dzero(c, 256 * sizeof(int));
    return c;
 }
+static int *defer_counter() { return device_flags() + 512 + 16; }
 
 // inclusive prefix sum over the 64 lanes of a wave
 __device__ __forceinline__ int wave_incl_scan(int v, int lane)
@@ -1037,8 +1040,10 @@ __global__ void k_pmis_remove(int nw, const int *__restrict__ list, const int *_
 // stay 1, everything else is 0 or -1), so the concurrent updates are safe.
 template <int K>
 __global__ void k_pmis_cf(int nw, const int *__restrict__ list, const int *__restrict__ S_ia,
-                          const int *__restrict__ S_ja, const double *__restrict__ m, int *CF)
+                          const int *__restrict__ S_ja, const double *__restrict__ m, int *CF,
+                          int *remaining)
 {
+   if (blockIdx.x == 0 && threadIdx.x == 0) { *remaining = 0; }   // counted by the update after this
    const int gl = threadIdx.x & (K - 1);
    const int rows_per_block = blockDim.x / K;
    const int gshift = (threadIdx.x & 63) & ~(K - 1);
@@ -1132,6 +1137,107 @@ __global__ __launch_bounds__(256) void k_pmis_update(int nw, const int *__restri
    }
 }
 
+// All rounds that are left once at most PM_FINISH rows are in the graph, by one
+// block with the list in LDS: a round of three kernels and a read-back takes
+// some 23 us whatever its rows, and half of a level's rounds have few.  The
+// passes are those of k_pmis_remove, k_pmis_cf and k_pmis_update, eight lanes a
+// row, with a barrier between; *rounds_out counts them (-1: no end).
+constexpr int PM_FINISH = 1024;
+
+__global__ __launch_bounds__(PM_FINISH) void k_pmis_finish(int nw, const int *__restrict__ list,
+                                                           const int *__restrict__ S_ia,
+                                                           const int *__restrict__ S_ja, double *m,
+                                                           int *CF, bool pick, int *rounds_out)
+{
+   constexpr int K = 8, RPB = PM_FINISH / K;
+   __shared__ int rows[2][PM_FINISH];
+   __shared__ int left;
+   const int gl = threadIdx.x & (K - 1), g = threadIdx.x / K;
+   const int gshift = (threadIdx.x & 63) & ~(K - 1);
+   if ((int) threadIdx.x < nw) { rows[0][threadIdx.x] = list ? list[threadIdx.x] : (int) threadIdx.x; }
+   __syncthreads();
+   int rounds = 0;
+   for (int cur = 0; nw > 0; cur ^= 1) {
+      if (++rounds > 100000) {
+         rounds = -1;
+         break;
+      }
+      for (int rb = 0; pick && rb < nw; rb += RPB) {
+         const bool act = rb + g < nw;
+         const int i = act ? rows[cur][rb + g] : 0;
+         const double mi = act ? m[i] : 0.0;
+         const bool cand = mi > 1;
+         const int s = cand ? S_ia[i] : 0, e = cand ? S_ia[i + 1] : 0;
+         const int klast = max(e - 1, 0);
+         bool lose = false;
+         for (int kb = s; __any(kb < e); kb += PM_U * K) {
+            int jv[PM_U];
+            double mv[PM_U];
+#pragma unroll
+            for (int u = 0; u < PM_U; u++) { jv[u] = S_ja[min(kb + gl + u * K, klast)]; }
+#pragma unroll
+            for (int u = 0; u < PM_U; u++) { mv[u] = m[jv[u]]; }
+#pragma unroll
+            for (int u = 0; u < PM_U; u++) {
+               if (kb + gl + u * K < e && mv[u] > 1) {
+                  if (mi > mv[u]) { CF[jv[u]] = 0; }
+                  else if (mv[u] > mi) { lose = true; }
+               }
+            }
+         }
+         if (((__ballot(lose) >> gshift) & 0xffull) && gl == 0) { CF[i] = 0; }
+      }
+      pick = true;
+      if (threadIdx.x == 0) { left = 0; }
+      __syncthreads();
+      for (int rb = 0; rb < nw; rb += RPB) {
+         const bool act = rb + g < nw;
+         const int i = act ? rows[cur][rb + g] : 0;
+         const double mi = act ? m[i] : 0.0;
+         const bool in_graph = act && mi > 0;
+         int c = in_graph ? CF[i] : 0;
+         if (in_graph && mi < 1) { c = -1; }
+         const bool scan = in_graph && !(c > 0);
+         const int s = scan ? S_ia[i] : 0, e = scan ? S_ia[i + 1] : 0;
+         const int klast = max(e - 1, 0);
+         bool hitc = false;
+         for (int kb = s; __any(kb < e); kb += PM_U * K) {
+            int jv[PM_U], cv[PM_U];
+#pragma unroll
+            for (int u = 0; u < PM_U; u++) { jv[u] = S_ja[min(kb + gl + u * K, klast)]; }
+#pragma unroll
+            for (int u = 0; u < PM_U; u++) { cv[u] = CF[jv[u]]; }
+#pragma unroll
+            for (int u = 0; u < PM_U; u++) {
+               if (kb + gl + u * K < e && cv[u] > 0) { hitc = true; }
+            }
+         }
+         const bool hm = ((__ballot(hitc) >> gshift) & 0xffull) != 0;
+         if (in_graph && gl == 0) {
+            if (c > 0) { c = 1; } else if (hm) { c = -1; }
+            CF[i] = c;
+         }
+      }
+      __syncthreads();
+      if ((int) threadIdx.x < nw) {
+         const int i = rows[cur][threadIdx.x];
+         const double mi = m[i];
+         if (mi > 0) {
+            if (CF[i] != 0) {
+               m[i] = 0.0;
+            } else {
+               if (mi > 1) { CF[i] = 1; }
+               rows[cur ^ 1][atomicAdd(&left, 1)] = i;
+            }
+         }
+      }
+      __syncthreads();
+      nw = left;
+      __syncthreads();
+   }
+   if (threadIdx.x == 0) { *rounds_out = rounds; }
+}
+
 int pmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_keep_dev,
          const int *st_count, int cf_init)
 {
@@ -1167,7 +1273,16 @@ int pmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_ke
    const int *list = nullptr;
    int nw = n;
    while (true) {
-      dzero(remaining, sizeof(int));
+      if (nw <= PM_FINISH) {
+         // what is left, in all its rounds, by one block
+         k_pmis_finish<<<1, PM_FINISH, 0, st>>>(nw, list, S.ia, S.ja, m, CF,
+                                               !(cf_init != 0 && rounds == 0), h);
+         HX_LAUNCH_CHECK();
+         sync();
+         if (h[0] < 0) { fail(HYPRE_ERROR_GENERIC, "PMIS did not terminate"); }
+         rounds += h[0];
+         break;
+      }
       const int nbk = (int) std::max<long long>(1, std::min<long long>(((long long) nw * K + 255) / 256, 16384));
       const int nbu = std::max(1, std::min((nw + 255) / 256, 8192));
       // par_coarsen.c:2487: with CF_init 1 the first round keeps the given
@@ -1175,7 +1290,7 @@ int pmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_ke
       const bool pick = !(cf_init != 0 && rounds == 0);
       dispatch_k(K, [&](auto kc) {
          if (pick) { k_pmis_remove<decltype(kc)::value><<<nbk, 256, 0, st>>>(nw, list, S.ia, S.ja, m, CF); }
-         k_pmis_cf<decltype(kc)::value><<<nbk, 256, 0, st>>>(nw, list, S.ia, S.ja, m, CF);
+         k_pmis_cf<decltype(kc)::value><<<nbk, 256, 0, st>>>(nw, list, S.ia, S.ja, m, CF, remaining);
       });
       int *next = lists[rounds & 1];
       k_pmis_update<<<nbu, 256, 0, st>>>(nw, list, m, CF, next, remaining);
@@ -3228,9 +3343,8 @@ void extpi_interp(const Csr &A, const Csr &S, int *CF, const int *f2c, int nc,
          f.raw_a = dalloc_n<double>((size_t) nwork * mc);
          f.cnt = raw_cnt;
          f.defer_list = lists[pass & 1];
-         f.ndefer = device_flags() + 60;
+         f.ndefer = defer_counter();
          f.claim = claim_counters();
-         dzero(f.ndefer, sizeof(int));
          const int nbt = (int) std::max<long long>(1, std::min<long long>((nwork + TR_ROWS - 1) / TR_ROWS, 16384));
          if (kind == 3) {
             k_extpi_rowg<16, XF_MC / 2><<<launch_blocks((nwork + 3) / 4), WAVE, 0, stream()>>>(f);
@@ -4499,7 +4613,7 @@ void rap(const Csr &R, const Csr &A, const Csr &P, Csr &Ac, int p_row_bound, int
    int *tj[3] = {nullptr, nullptr, nullptr};
    double *ta[3] = {nullptr, nullptr, nullptr};
    int *lists[2] = {dalloc_n<int>((size_t) nc + 1), dalloc_n<int>((size_t) nc + 1)};
-   int *ndefer = device_flags() + 60;
+   int *ndefer = defer_counter();
    int *h = static_cast<int *>(pinned_scratch(64));
    f.cnt = cnt;
    f.src = src;
@@ -4541,7 +4655,6 @@ void rap(const Csr &R, const Csr &A, const Csr &P, Csr &Ac, int p_row_bound, int
       f.tmp_j = tj[stage];
       f.tmp_a = ta[stage];
       f.defer_list = lists[cur];
-      dzero(ndefer, sizeof(int));
       f.claim = claim_counters();
       if (raregs[stage] > 0) { f.rcl = raregs[stage] * WAVE; }
       const size_t lds = rap_fast_lds(f.rc, f.rcl, f.ac, f.acl, raregs[stage]);

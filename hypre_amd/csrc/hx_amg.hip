@@ -125,22 +125,37 @@ void AMGSolver::setup(const Csr &A0)
       side_after_main();
       probed = sten_probe(A0, L[0].sten, 4096, side_stream());
    }
-   // the full values of the slices that need them, once the fill has said so
-   auto finish_sten = [&]() {
-      if (L[0].sten.nslices <= 0 || L[0].sten.raw) { return; }
+   // start_sten: the copy's fill, once the probe has ended, beside the fine
+   // level's PMIS; finish_sten: the full values of the slices that need them
+   // (before interpolation, which reads the copy)
+   auto start_sten = [&]() {
+      if (!probed) { return; }
+      probed = false;
       side_sync();
-      if (sten_raw_slices() > 0) {
+      if (sten_take(L[0].sten)) {
          side_after_main();
-         sten_fill_raw(A0, L[0].sten, p.cycle_fp32 != 0, side_stream());
+         sten_fill(A0, L[0].sten, side_stream());
       }
+   };
+   auto finish_sten = [&]() {
+      Sten &st = L[0].sten;
+      if (st.nslices <= 0) { return; }
+      side_sync();
+      sten_counts(st);
+      if (st.tab.raw > 0 && !st.raw) {
+         side_after_main();
+         sten_fill_raw(A0, st, p.cycle_fp32 != 0, side_stream());
+      }
+      main_after_side();
    };
    auto start_ell = [&](int j) {
       Level &lv = L[j];
-      if (j == 0 && probed) {
-         side_sync();
-         if (sten_take(lv.sten)) {
-            side_after_main();
-            sten_fill(A0, lv.sten, side_stream());
+      if (j == 0) {
+         if (probed) {
+            start_sten();
+            finish_sten();
+         }
+         if (lv.sten.nslices > 0) {
             ell_started = 1;
             return;
          }
@@ -175,6 +190,7 @@ void AMGSolver::setup(const Csr &A0)
          create_s(A, theta(level), p.max_row_sum, lv.S, stc, lv.l1, l1_zero_flag(level), s_thr,
                   s_flg, level == 0);
       }
+      if (level == 0) { start_sten(); }
       lv.CF = dalloc_n<int>((size_t) fine_size);
       if (p.keep_setup_data) { lv.measure = dalloc_n<double>((size_t) fine_size); }
       {
@@ -208,6 +224,7 @@ void AMGSolver::setup(const Csr &A0)
          S2.free_all();
       }
       const int coarse_size = coarse_map(fine_size, lv.CF, f2c);
+      if (level == 0) { finish_sten(); }
       // par_amg_setup.c:1690-1725
       if (coarse_size == 0 || coarse_size == fine_size) {
          if (coarse_relax == 9 || coarse_relax == 19 || coarse_relax == 98 || coarse_relax == 99) {
@@ -235,7 +252,7 @@ void AMGSolver::setup(const Csr &A0)
       } else {
          Range r("ExtPIInterp");   // par_lr_interp.c:5564
          extpi_interp(A, lv.S, lv.CF, f2c, coarse_size, p.trunc_factor, p.P_max_elmts, lv.P, s_thr,
-                      s_flg);
+                      s_flg, &lv.sten);
       }
       dfree(s_thr);
       dfree(s_flg);
@@ -256,7 +273,6 @@ void AMGSolver::setup(const Csr &A0)
          rap(cur.R, *cur.A, cur.P, nx.Aown, pmx > 0 ? std::max(pmx, 1) : 0, a_max_row,
              &a_max_row);
       }
-      if (level == 0) { finish_sten(); }
       nx.A = &nx.Aown;
       level++;
       // par_amg_setup.c:3136-3141 (the host-only switch to CLJP coarsening
@@ -350,9 +366,7 @@ void AMGSolver::setup(const Csr &A0)
          }
       }
    }
-   const bool late = ell_started == 0;
    for (int j = ell_started; j < num_levels; j++) { start_ell(j); }
-   if (late) { finish_sten(); }
    // the solve phase runs after the copies are filled
    main_after_side();
    for (int j = 0; j < num_levels; j++) {

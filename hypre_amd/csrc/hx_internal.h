@@ -161,9 +161,20 @@ struct Ell
 // then ascending; 0 past the D-th) and the value of one entry of each
 struct StenHead
 {
-   int    ok, D, wmax, raw;       // raw: slices whose values are kept in full
+   int    ok, D, wmax;            // stencil or not, offsets, longest row
+   int    raw, coded;             // slices with full values, with a dictionary
+   int    hops;                   // distinct sums of two offsets
    int    off[32];
    double v[32];
+};
+constexpr int STEN_HOPS = 128;    // most sums that StenHop lists
+// The sums of two offsets: entry l of row i + off[k] is column
+// i + hop[id[k * 32 + l]]; mirror[k]: the step of -off[k], -1 if there is none
+struct StenHop
+{
+   int           mirror[32];
+   int           hop[STEN_HOPS];
+   unsigned char id[32 * 32];
 };
 
 // Stencil copy of an operator for the solve phase (hx_stencil.hip): one mask
@@ -175,6 +186,7 @@ struct Sten
    int       nslices = 0;         // 0: no copy
    int      *st = nullptr;        // probe's words
    StenHead *head = nullptr;
+   StenHop  *hop = nullptr;
    unsigned *mask = nullptr;      // bit k: the row has step k
    int      *info = nullptr;      // per slice: mode | 4 if all rows have all steps | values << 8
    unsigned *codes = nullptr;     // four codes a word, word w of 64 rows contiguous
@@ -209,13 +221,18 @@ void ell_fill(const Csr &A, Ell &E, bool fp32, hipStream_t s);
 // The stencil copy, in steps on stream s: sten_probe launches the search for
 // the offsets (false: not worth it for this operator), sten_take reads its
 // result once s has finished (false: no stencil), sten_fill builds the copy,
-// and sten_fill_raw, once s has finished and sten_raw_slices() says that some
-// slice needs it, the full values
+// and sten_fill_raw, once sten_counts says that some slice needs it, the full
+// values
 bool sten_probe(const Csr &A, Sten &S, int min_rows, hipStream_t s);
 bool sten_take(Sten &S);
 void sten_fill(const Csr &A, Sten &S, hipStream_t s);
-int  sten_raw_slices();
+// the counts of slices, into S.tab, once s has finished the fill
+void sten_counts(Sten &S);
 void sten_fill_raw(const Csr &A, Sten &S, bool fp32, hipStream_t s);
+// Per row of A, as step masks: x strong entries (thr, flg as create_s keeps
+// them), y neighbours that are C points, z neighbours with CF -3, w entries of
+// the sign opposite to the diagonal's
+void sten_masks(const Csr &A, const Sten &S, const double *thr, const int *flg, const int *CF, uint4 *q);
 template <typename V, typename X, bool DOT>
 int sten_spmv(const Csr &A, X alpha, const X *x, X beta, const X *b, X *y, double *part);
 template <typename V, typename X>
@@ -341,10 +358,11 @@ void rs_first_pass_host(int n, const int *S_ia, const int *S_ja, int *CF);
 int  coarse_map(int n, const int *CF, int *f2c);
 // ext+i interpolation + truncation (CF: -3 -> -1 on exit)
 // s_thr / s_flg: the strength thresholds and flags create_s produced for S
-// (optional; they let the C lists be built in one pass over A)
+// (optional; they let the C lists be built in one pass over A); sten: A's
+// filled stencil copy (optional; needs both)
 void extpi_interp(const Csr &A, const Csr &S, int *CF, const int *f2c, int nc,
                   double trunc_factor, int max_elmts, Csr &P, const double *s_thr = nullptr,
-                  const int *s_flg = nullptr);
+                  const int *s_flg = nullptr, const Sten *sten = nullptr);
 // hypre_BoomerAMGInterpTruncation of P in place (rows of <= 64 entries)
 void truncate_rows(Csr &P, double trunc_factor, int max_elmts);
 // aggressive coarsening: the second strength matrix over the nc C points of

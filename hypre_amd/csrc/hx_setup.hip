@@ -3102,11 +3102,22 @@ __device__ void qsort2_abs_strided(unsigned char *v, double *w, int cnt, int kee
         double tw = w[left * SS]; w[left * SS] = w[mid * SS]; w[mid * SS] = tw; }
       int last = left;
       const double piv = fabs(w[left * SS]);
-      for (int i = left + 1; i <= right; i++) {
-         if (fabs(w[i * SS]) > piv) {
-            ++last;
-            unsigned char t = v[last * SS]; v[last * SS] = v[i * SS]; v[i * SS] = t;
-            double tw = w[last * SS]; w[last * SS] = w[i * SS]; w[i * SS] = tw;
+      // four values ahead: an exchange touches no place past the value it is for
+      for (int i = left + 1; i <= right; i += 4) {
+         double wi[4];
+#pragma unroll
+         for (int u = 0; u < 4; u++) { wi[u] = w[min(i + u, right) * SS]; }
+#pragma unroll
+         for (int u = 0; u < 4; u++) {
+            if (i + u <= right && fabs(wi[u]) > piv) {
+               ++last;
+               const unsigned char t = v[last * SS], vi = v[(i + u) * SS];
+               const double tw = w[last * SS];
+               v[last * SS] = vi;
+               v[(i + u) * SS] = t;
+               w[last * SS] = wi[u];
+               w[(i + u) * SS] = tw;
+            }
          }
       }
       { unsigned char t = v[left * SS]; v[left * SS] = v[last * SS]; v[last * SS] = t;
@@ -3131,6 +3142,55 @@ __device__ void qsort2_abs_strided(unsigned char *v, double *w, int cnt, int kee
          sp++;
       }
    }
+}
+
+// The truncation of one row of c entries in LDS (values vw, payload bytes vj,
+// stride SS); returns how many are left, in the first places.
+template <int SS>
+__device__ int trunc_row(unsigned char *vj, double *vw, int c, double trunc_factor, int max_elmts)
+{
+   int kept = c;
+   if (trunc_factor > 0) {
+      double row_nrm = 0.0;
+      for (int k = 0; k < c; k++) {
+         const double a = fabs(vw[k * SS]);
+         row_nrm = (row_nrm < a) ? a : row_nrm;
+      }
+      const double drop_coeff = trunc_factor * row_nrm;
+      double row_sum = 0.0, scale = 0.0;
+      int o = 0;
+      for (int k = 0; k < c; k++) {
+         const double w = vw[k * SS];
+         row_sum += w;
+         if (fabs(w) < drop_coeff) { continue; }
+         scale += w;
+         vw[o * SS] = w;
+         vj[o * SS] = vj[k * SS];
+         o++;
+      }
+      if (scale != 0.) {
+         if (scale != row_sum) {
+            scale = row_sum / scale;
+            for (int k = 0; k < o; k++) { vw[k * SS] *= scale; }
+         }
+      }
+      kept = o;
+   }
+   if (max_elmts > 0 && kept > max_elmts) {
+      double row_sum = 0.0;
+      for (int k = 0; k < kept; k++) { row_sum += vw[k * SS]; }
+      qsort2_abs_strided<SS>(vj, vw, kept, max_elmts);
+      double scale = 0.0;
+      for (int k = 0; k < max_elmts; k++) { scale += vw[k * SS]; }
+      if (scale != 0.) {
+         if (scale != row_sum) {
+            scale = row_sum / scale;
+            for (int k = 0; k < max_elmts; k++) { vw[k * SS] *= scale; }
+         }
+      }
+      kept = max_elmts;
+   }
+   return kept;
 }
 
 // par_csr_matrix.c:3040-3320 (trunc_factor drop + rescale, then P_max_elmts
@@ -3191,47 +3251,7 @@ __global__ __launch_bounds__(TR_ROWS) void k_trunc_rows(int n, const int *__rest
       if (c >= 0) {
          unsigned char *vj = sv + t;
          double *vw = sw + t;
-         int kept = c;
-         if (trunc_factor > 0) {
-            double row_nrm = 0.0;
-            for (int k = 0; k < c; k++) {
-               const double a = fabs(vw[k * TR_SS]);
-               row_nrm = (row_nrm < a) ? a : row_nrm;
-            }
-            const double drop_coeff = trunc_factor * row_nrm;
-            double row_sum = 0.0, scale = 0.0;
-            int o = 0;
-            for (int k = 0; k < c; k++) {
-               const double w = vw[k * TR_SS];
-               row_sum += w;
-               if (fabs(w) < drop_coeff) { continue; }
-               scale += w;
-               vw[o * TR_SS] = w;
-               vj[o * TR_SS] = vj[k * TR_SS];
-               o++;
-            }
-            if (scale != 0.) {
-               if (scale != row_sum) {
-                  scale = row_sum / scale;
-                  for (int k = 0; k < o; k++) { vw[k * TR_SS] *= scale; }
-               }
-            }
-            kept = o;
-         }
-         if (max_elmts > 0 && kept > max_elmts) {
-            double row_sum = 0.0;
-            for (int k = 0; k < kept; k++) { row_sum += vw[k * TR_SS]; }
-            qsort2_abs_strided<TR_SS>(vj, vw, kept, max_elmts);
-            double scale = 0.0;
-            for (int k = 0; k < max_elmts; k++) { scale += vw[k * TR_SS]; }
-            if (scale != 0.) {
-               if (scale != row_sum) {
-                  scale = row_sum / scale;
-                  for (int k = 0; k < max_elmts; k++) { vw[k * TR_SS] *= scale; }
-               }
-            }
-            kept = max_elmts;
-         }
+         const int kept = trunc_row<TR_SS>(vj, vw, c, trunc_factor, max_elmts);
          const long long row = rowlist ? rowlist[i] : i;
          out_cnt[row] = kept;
          const int *rj = raw_j + (size_t) i * MC;
@@ -3281,9 +3301,319 @@ __global__ void k_cf_fix(int n, int *CF)
    }
 }
 
+// ------------------------------------------------------------------ ext+i on a stencil operator
+// One lane a row, truncation included, for operators with a stencil copy whose
+// two-hop columns are at most STEN_HOPS distinct offsets from the row (125 for
+// 27 points, 25 for 7).  Which column a neighbour's entry is, is then
+// arithmetic: step k of the row and step l of its neighbour name a hop, and a
+// byte per hop and lane says where the hop stands in C-hat.  The kernels above
+// find the same out with a hash of columns, some 700 wave instructions a row.
+// Neighbours' masks are loads at scalar bases; steps run in the wave's common
+// order, which is every row's storage order, so C-hat, weights, denominators
+// and diagonals get their terms in hypre's order.  CONSTV: all values are the
+// table's; otherwise a neighbour's entry is looked up in its CSR row (its rank
+// is the mask's bits below it).  Rows with more than MC C-hat points are handed
+// on.  Bound by instruction issue (the wave takes as many terms a step as its
+// longest list, five or six where the mean is two) and by 8 waves a CU, which
+// the 19 KB of LDS allow.  Measured and dropped: C-hat as a bit set in
+// registers with ranks by population counts (9 waves a CU, four times the
+// instructions a term: 8.3 ms), terms one at a time (8.2 ms).
+// Level 0 of 27-point 200^3, with masks and truncation: 11.2 + 1.9 + 1.4 ms of
+// separate kernels -> 5.0 + 0.3; jumping coefficients 320^3 55 -> 31 ms.
+struct ExtpiStenArgs
+{
+   int             n, D, hops;
+   const uint4    *q;           // step masks (sten_masks)
+   const unsigned *mask;
+   const StenHead *tab;
+   const StenHop  *hop;
+   const int      *A_ia;
+   const double   *A_a;
+   const int      *CF, *f2c;
+   double          trunc_factor;
+   int             max_elmts;
+   int            *out_cnt, *out_j;
+   double         *out_a;
+   const int      *rowlist;     // rows to process (nullptr: all)
+   int             nwork;
+   int            *defer_list, *ndefer;
+};
+
+static size_t extpi_sten_lds(int MC, int hops)
+{
+   return sizeof(double) * ((size_t) MC * WAVE + 32) + sizeof(int) * STEN_HOPS + 32 * 32 +
+          (size_t) MC * WAVE + (size_t) hops * WAVE;
+}
+
+template <int MC, bool CONSTV>
+__global__ __launch_bounds__(WAVE) void k_extpi_sten(ExtpiStenArgs p)
+{
+   extern __shared__ __align__(16) char lds_sten[];
+   double *wgt = reinterpret_cast<double *>(lds_sten);            // [MC][lane]
+   double *vt = wgt + MC * WAVE;
+   int *hop = reinterpret_cast<int *>(vt + 32);
+   unsigned char *id = reinterpret_cast<unsigned char *>(hop + STEN_HOPS);
+   unsigned char *pos = id + 32 * 32;                             // [hop][lane]: place in C-hat
+   unsigned char *list = pos + p.hops * WAVE;                     // [MC][lane]: hops of C-hat
+   constexpr int NONE = 0xff;
+   const int lane = threadIdx.x, D = p.D, n = p.n;
+   for (int i = lane; i < 32; i += WAVE) { vt[i] = p.tab->v[i]; }
+   for (int i = lane; i < p.hops; i += WAVE) { hop[i] = p.hop->hop[i]; }
+   for (int i = lane; i < 32 * 32; i += WAVE) { id[i] = p.hop->id[i]; }
+   wave_sync();
+   // blocks of an XCD take every nbx-th group of 64 rows of its share
+   const int nr = p.rowlist ? p.nwork : n;
+   const int ng = (nr + WAVE - 1) / WAVE;
+   const int nx = (gridDim.x & 7) ? 1 : 8, nbx = gridDim.x / nx;
+   const int share = (ng + nx - 1) / nx;
+   const long long first = (long long) (blockIdx.x % nx) * share;
+   const int g1 = (int) min((long long) ng, first + share);
+   for (long long g = first + blockIdx.x / nx; g < g1; g += nbx) {
+      const int w = (int) g * WAVE + lane;
+      const bool valid = w < nr;
+      const int i = valid ? (p.rowlist ? p.rowlist[w] : w) : n - 1;
+      const int cf = valid ? p.CF[i] : -3;
+      if (valid && cf >= 0) {
+         p.out_cnt[i] = 1;
+         p.out_j[(size_t) i * p.max_elmts] = p.f2c[i];
+         p.out_a[(size_t) i * p.max_elmts] = 1.0;
+      } else if (valid && cf == -3) {
+         p.out_cnt[i] = 0;
+      }
+      bool live = valid && cf < 0 && cf != -3;
+      if (!__any(live)) { continue; }
+      uint4 q = {0u, 0u, 0u, 0u};
+      unsigned am = 0u;
+      int ia = 0;
+      if (live) {
+         q = p.q[i];
+         am = p.mask[i];
+         ia = p.A_ia[i];
+      }
+      for (int t = lane; t < p.hops * (WAVE / 16); t += WAVE) {
+         reinterpret_cast<uint4 *>(pos)[t] = uint4{~0u, ~0u, ~0u, ~0u};
+      }
+      wave_sync();
+      // rows outside [0, n) belong to steps that the row does not have
+      auto nb = [&](int k) { return max(0, min(n - 1, i + p.tab->off[k])); };
+      // C-hat (par_lr_interp.c:1505-1560): a strong C neighbour is step 0 of
+      // its own row, a strong F neighbour brings its strong C points
+      int nch = 0;
+      uint2 qn = *reinterpret_cast<const uint2 *>(p.q + nb(min(1, D - 1)));
+      for (int k = 1; k < D; k++) {
+         const uint2 c = qn;
+         if (k + 1 < D) { qn = *reinterpret_cast<const uint2 *>(p.q + nb(k + 1)); }
+         unsigned bits = 0u;
+         if (q.x >> k & 1u) {
+            if (q.y >> k & 1u) { bits = 1u; }
+            else if (!(q.z >> k & 1u)) { bits = c.x & c.y; }
+         }
+         // three at a time: a row's columns are distinct
+         while (__any(bits != 0u)) {
+            int t[3], at[3];
+            bool in[3];
+#pragma unroll
+            for (int u = 0; u < 3; u++) {
+               in[u] = bits != 0u;
+               t[u] = id[k * 32 + max(__ffs((int) bits) - 1, 0)];
+               bits &= bits - 1u;
+            }
+#pragma unroll
+            for (int u = 0; u < 3; u++) { at[u] = pos[t[u] * WAVE + lane]; }
+#pragma unroll
+            for (int u = 0; u < 3; u++) {
+               if (in[u] && at[u] == NONE) {
+                  if (nch < MC) {
+                     pos[t[u] * WAVE + lane] = (unsigned char) nch;
+                     list[nch * WAVE + lane] = (unsigned char) t[u];
+                  }
+                  nch++;
+               }
+            }
+         }
+      }
+      if (live && nch > MC) {
+         live = false;
+         p.out_cnt[i] = -1;
+         p.defer_list[atomicAdd(p.ndefer, 1)] = i;
+      }
+      if (!live) { am = 0u; }
+      for (int c = 0; __any(live && c < nch); c++) { wgt[c * WAVE + lane] = 0.0; }
+      // weights and the diagonal (par_lr_interp.c:1640-1800)
+      double diag = 0.0, an = 0.0;
+      unsigned mn = 0u;
+      int jn = 0;
+      uint4 qw = {0u, 0u, 0u, 0u};
+      auto load = [&](int k) {
+         const int j = nb(k);
+         qw = p.q[j];
+         if (!CONSTV) {
+            mn = p.mask[j];
+            jn = p.A_ia[j];
+            an = p.A_a[ia + ((am >> k & 1u) ? __popc(am & ((1u << k) - 1u)) : 0)];
+         }
+      };
+      if (live) { diag = CONSTV ? vt[0] : p.A_a[ia]; }
+      load(min(1, D - 1));
+      for (int k = 1; k < D; k++) {
+         const uint4 c = qw;
+         const unsigned m1 = mn;
+         const int a1 = jn;
+         const double aij = CONSTV ? vt[k] : an;
+         if (k + 1 < D) { load(k + 1); }
+         const bool has = am >> k & 1u;
+         if (!__any(has)) { continue; }
+         const int lm = p.hop->mirror[k];
+         unsigned bits = 0u;
+         bool self = false, open = false;
+         if (has) {
+            const int at = pos[id[k * 32] * WAVE + lane];
+            if (at != NONE) {
+               wgt[at * WAVE + lane] += aij;
+            } else if ((q.x >> k & 1u) && !((q.y | q.z) >> k & 1u)) {
+               open = true;
+               self = lm >= 0 && (c.w >> lm & 1u);
+               bits = c.w & c.y;
+            } else if (!(q.z >> k & 1u)) {
+               diag += aij;   // weak connection
+            }
+         }
+         if (!__any(open)) { continue; }
+         // the terms of row i + off[k] that lie in C-hat, in its storage order:
+         // places and values of U at a time, the first two batches kept (a
+         // wave's longest list has five or six); column i's term comes in
+         // where its step does
+         constexpr int U = 3;
+         const double sai = self ? (CONSTV ? vt[max(lm, 0)] : p.A_a[a1 + __popc(m1 & ((1u << lm) - 1u))]) : 0.0;
+         int to[2][U];
+         double v[2][U];
+         double sum = 0.0;
+         bool pend = self;
+         auto batch = [&](unsigned &rest, int (&tb)[U], double (&vb)[U], bool fold) {
+            int l[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+               l[u] = __ffs((int) rest) - 1;   // -1 past the last
+               rest &= rest - 1u;
+               const int lc = max(l[u], 0);
+               tb[u] = id[k * 32 + lc];
+               vb[u] = CONSTV ? vt[lc] : p.A_a[a1 + __popc(m1 & ((1u << lc) - 1u))];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+               const int at = pos[tb[u] * WAVE + lane];
+               tb[u] = l[u] >= 0 ? at : NONE;
+            }
+            if (fold) {
+#pragma unroll
+               for (int u = 0; u < U; u++) {
+                  if (tb[u] != NONE) {
+                     if (pend && lm < l[u]) {
+                        sum += sai;
+                        pend = false;
+                     }
+                     sum += vb[u];
+                  }
+               }
+            }
+         };
+         unsigned rest = bits;
+         batch(rest, to[0], v[0], true);
+         const bool two = __any(rest != 0u);
+         bool more = false;
+         unsigned tail = 0u;
+         if (two) {
+            batch(rest, to[1], v[1], true);
+            tail = rest;
+            more = __any(rest != 0u);
+            while (__any(rest != 0u)) {
+               int tx[U];
+               double vx[U];
+               batch(rest, tx, vx, true);
+            }
+         }
+         if (pend) { sum += sai; }
+         const bool ok = open && sum != 0.0;
+         if (open && !ok) { diag += aij; }
+         const double dist = ok ? aij / sum : 0.0;
+         if (ok && self) { diag += dist * sai; }
+         // a row's columns are distinct: a batch's weights are read, then written
+         auto spread = [&](const int (&tb)[U], const double (&vb)[U]) {
+            double x[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) { x[u] = wgt[(tb[u] & (MC - 1)) * WAVE + lane]; }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+               if (ok && tb[u] != NONE) { wgt[tb[u] * WAVE + lane] = x[u] + dist * vb[u]; }
+            }
+         };
+         spread(to[0], v[0]);
+         if (two) { spread(to[1], v[1]); }
+         if (more) {
+            while (__any(tail != 0u)) {
+               int tx[U];
+               double vx[U];
+               batch(tail, tx, vx, false);
+               spread(tx, vx);
+            }
+         }
+      }
+      if (live) {
+         if (diag != 0.0) {
+            for (int c = 0; c < nch; c++) { wgt[c * WAVE + lane] /= -diag; }
+         }
+         const int kept = trunc_row<WAVE>(list + lane, wgt + lane, nch, p.trunc_factor, p.max_elmts);
+         p.out_cnt[i] = kept;
+         for (int c = 0; c < kept; c++) {
+            p.out_j[(size_t) i * p.max_elmts + c] = p.f2c[i + hop[list[c * WAVE + lane]]];
+            p.out_a[(size_t) i * p.max_elmts + c] = wgt[c * WAVE + lane];
+         }
+      }
+      wave_sync();
+   }
+}
+
+// the passes over a stencil operator, 16 C-hat points a row, then 32 for the
+// few rows that have more; returns the number of rows handed on (in lists[1])
+static int extpi_sten(const Csr &A, const Sten &S, const int *CF, const int *f2c, double trunc_factor,
+                      int max_elmts, const double *thr, const int *flg, int *cnt, int *out_j,
+                      double *out_a, int *const *lists)
+{
+   uint4 *q = dalloc_n<uint4>((size_t) A.nrows);
+   sten_masks(A, S, thr, flg, CF, q);
+   ExtpiStenArgs p{};
+   p.n = A.nrows; p.D = S.tab.D; p.hops = S.tab.hops;
+   p.q = q; p.mask = S.mask; p.tab = S.head; p.hop = S.hop;
+   p.A_ia = A.ia; p.A_a = A.a; p.CF = CF; p.f2c = f2c;
+   p.trunc_factor = trunc_factor; p.max_elmts = max_elmts;
+   p.out_cnt = cnt; p.out_j = out_j; p.out_a = out_a;
+   p.ndefer = defer_counter();
+   const bool all_const = S.tab.raw == 0 && S.tab.coded == 0;
+   int left = A.nrows;
+   for (int pass = 0; pass < 2 && left > 0; pass++) {
+      p.rowlist = pass ? lists[0] : nullptr;
+      p.nwork = left;
+      p.defer_list = lists[pass];
+      dzero(p.ndefer, sizeof(int));
+      const size_t lds = extpi_sten_lds(pass ? 32 : 16, S.tab.hops);
+      const int nb = resident_blocks(((long long) left + WAVE - 1) / WAVE, lds);
+      if (pass == 0 && all_const) { k_extpi_sten<16, true><<<nb, WAVE, lds, stream()>>>(p); }
+      else if (pass == 0) { k_extpi_sten<16, false><<<nb, WAVE, lds, stream()>>>(p); }
+      else if (all_const) { k_extpi_sten<32, true><<<nb, WAVE, lds, stream()>>>(p); }
+      else { k_extpi_sten<32, false><<<nb, WAVE, lds, stream()>>>(p); }
+      HX_LAUNCH_CHECK();
+      d2h(&left, p.ndefer, sizeof(int));
+      if (setup_verbose()) {
+         std::fprintf(stderr, "[hypre_mi355x] ext+i %d rows, stencil pass %d: %d left\n", A.nrows, pass, left);
+      }
+   }
+   dfree(q);
+   return left;
+}
+
 void extpi_interp(const Csr &A, const Csr &S, int *CF, const int *f2c, int nc,
                   double trunc_factor, int max_elmts, Csr &P, const double *s_thr,
-                  const int *s_flg)
+                  const int *s_flg, const Sten *sten)
 {
    int n = A.nrows;
    TimedLaunch tl("setup_interp", 0.0);
@@ -3302,8 +3632,18 @@ void extpi_interp(const Csr &A, const Csr &S, int *CF, const int *f2c, int nc,
    if (max_elmts > 0 && max_elmts <= XF_MC) {
       // fast path into raw rows, truncation per thread, leftovers by k_extpi
       stride = max_elmts;
+      tmp_j = dalloc_n<int>((size_t) std::max(n, 1) * stride);
+      tmp_a = dalloc_n<double>((size_t) std::max(n, 1) * stride);
+      int *lists[2] = {dalloc_n<int>((size_t) n + 1), dalloc_n<int>((size_t) n + 1)};
+      const int *list = nullptr;
+      int nwork = n;
+      if (sten && sten->nslices > 0 && s_thr && s_flg && sten->tab.hops <= STEN_HOPS) {
+         nwork = extpi_sten(A, *sten, CF, f2c, trunc_factor, max_elmts, s_thr, s_flg, cnt, tmp_j, tmp_a,
+                            lists);
+         list = lists[1];
+      }
       CLists CL;
-      c_lists(A, S, CF, CL, s_thr, s_flg);
+      if (nwork > 0) { c_lists(A, S, CF, CL, s_thr, s_flg); }
       ExtpiFastArgs f{};
       f.n = n;
       f.A_ia = A.ia; f.A_ja = A.ja; f.A_a = A.a;
@@ -3311,12 +3651,7 @@ void extpi_interp(const Csr &A, const Csr &S, int *CF, const int *f2c, int nc,
       f.SC_cnt = CL.sc_cnt; f.SC_ja = CL.sc_ja;
       f.OC_cnt = CL.oc_cnt; f.OC = CL.oc;
       f.CF = CF; f.f2c = f2c;
-      tmp_j = dalloc_n<int>((size_t) std::max(n, 1) * stride);
-      tmp_a = dalloc_n<double>((size_t) std::max(n, 1) * stride);
       int *h = static_cast<int *>(pinned_scratch(64));
-      int *lists[2] = {dalloc_n<int>((size_t) n + 1), dalloc_n<int>((size_t) n + 1)};
-      const int *list = nullptr;
-      int nwork = n;
       // passes over the rows left by the previous one: two rows per wave (rows
       // of <= 32 entries; tried where the mean row is that short), one row
       // per wave (C-hat <= 32 points; tried where the mean row has at most

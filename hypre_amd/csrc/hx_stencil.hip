@@ -152,6 +152,8 @@ __global__ __launch_bounds__(ST_SLOTS) void k_sten_table(const int *__restrict__
       out->D = ok ? st[1] : 0;
       out->wmax = st[2];
       out->raw = 0;
+      out->coded = 0;
+      out->hops = 0;
    }
    __syncthreads();
    if (!ok || key[i] == ST_EMPTY) { return; }
@@ -164,6 +166,41 @@ __global__ __launch_bounds__(ST_SLOTS) void k_sten_table(const int *__restrict__
       out->off[rank] = key[i];
       out->v[rank] = a[st[ST_REP + i]];
    }
+}
+
+// distinct sums of two offsets in ascending order, numbered for every pair, by
+// comparing all with all (on the side stream, beside the first setup kernels)
+__global__ __launch_bounds__(ST_MAX * ST_MAX) void k_sten_hop(StenHead *__restrict__ T,
+                                                             StenHop *__restrict__ out)
+{
+   __shared__ long long sum[ST_MAX * ST_MAX];
+   __shared__ unsigned char first[ST_MAX * ST_MAX];
+   __shared__ int count;
+   const int i = threadIdx.x, k = i / ST_MAX, l = i % ST_MAX;
+   const int D = T->D;
+   const bool in = T->ok && k < D && l < D;
+   const long long NONE = LLONG_MAX;
+   sum[i] = in ? (long long) T->off[k] + T->off[l] : NONE;
+   if (i == 0) { count = 0; }
+   __syncthreads();
+   bool f = in;
+   for (int j = 0; j < i; j++) { f = f && sum[j] != sum[i]; }
+   first[i] = f;
+   if (f) { atomicAdd(&count, 1); }
+   __syncthreads();
+   if (i == 0) { T->hops = count; }
+   if (i < ST_MAX) {
+      int m = -1;
+      for (int j = 0; j < D; j++) {
+         if (i < D && T->off[j] == -T->off[i]) { m = j; }
+      }
+      out->mirror[i] = m;
+   }
+   if (!in || count > STEN_HOPS) { return; }
+   int rank = 0;
+   for (int j = 0; j < ST_MAX * ST_MAX; j++) { rank += first[j] && sum[j] < sum[i]; }
+   out->id[i] = (unsigned char) rank;
+   if (f) { out->hop[rank] = (int) sum[i]; }
 }
 
 // ---------------------------------------------------------------- filling
@@ -208,7 +245,8 @@ __global__ __launch_bounds__(64) void k_sten_fill(int n, int ns, StenHead T,
                                                   unsigned *__restrict__ mask,
                                                   int *__restrict__ info,
                                                   unsigned *__restrict__ codes,
-                                                  double *__restrict__ dict, int *__restrict__ nraw)
+                                                  double *__restrict__ dict, int *__restrict__ nraw,
+                                                  int *__restrict__ ncoded)
 {
    __shared__ int sj[SF_CH];
    __shared__ double sa[SF_CH];
@@ -310,7 +348,10 @@ __global__ __launch_bounds__(64) void k_sten_fill(int n, int ns, StenHead T,
             dict[(size_t) sl * ST_DICT + num[i]] = __longlong_as_double((long long) key[i]);
          }
       }
-      if (lane == 0) { info[sl] = ST_CODES | fl | count << 8; }
+      if (lane == 0) {
+         info[sl] = ST_CODES | fl | count << 8;
+         atomicAdd(ncoded, 1);
+      }
    }
 }
 
@@ -350,7 +391,7 @@ __global__ __launch_bounds__(64) void k_sten_raw(int n, int ns, StenHead T,
 
 void Sten::free_all()
 {
-   dfree(st); dfree(head); dfree(mask); dfree(info); dfree(codes); dfree(dict); dfree(raw);
+   dfree(st); dfree(head); dfree(hop); dfree(mask); dfree(info); dfree(codes); dfree(dict); dfree(raw);
    dfree(raw32);
    *this = Sten();
 }
@@ -373,6 +414,7 @@ bool sten_probe(const Csr &A, Sten &S, int min_rows, hipStream_t s)
    }
    S.st = dalloc_n<int>(ST_WORDS);
    S.head = dalloc_n<StenHead>(1);
+   S.hop = dalloc_n<StenHop>(1);
    sten_pinned()->ok = 0;
    k_sten_init<<<1, BS, 0, s>>>(S.st);
    HX_LAUNCH_CHECK();
@@ -380,6 +422,8 @@ bool sten_probe(const Csr &A, Sten &S, int min_rows, hipStream_t s)
    k_sten_probe<<<nb, BS, 0, s>>>(A.nrows, A.ia, A.ja, S.st);
    HX_LAUNCH_CHECK();
    k_sten_table<<<1, ST_SLOTS, 0, s>>>(S.st, A.a, S.head);
+   HX_LAUNCH_CHECK();
+   k_sten_hop<<<1, ST_MAX * ST_MAX, 0, s>>>(S.head, S.hop);
    HX_LAUNCH_CHECK();
    HX_HIP(hipMemcpyAsync(sten_pinned(), S.head, sizeof(StenHead), hipMemcpyDeviceToHost, s));
    return true;
@@ -392,9 +436,9 @@ bool sten_take(Sten &S)
    return S.tab.ok != 0;
 }
 
-// One-wave blocks, four a CU: beside the level's RAP the copy takes a small
-// share of the CUs (the same grid as the sliced-ELL fill).
-constexpr int SF_GRID = 1024;
+// One-wave blocks, eight a CU (9 fit its LDS): the fill runs beside the fine
+// level's PMIS, short kernels and waits, and has to be done when they are.
+constexpr int SF_GRID = 2048;
 
 void sten_fill(const Csr &A, Sten &S, hipStream_t s)
 {
@@ -406,12 +450,16 @@ void sten_fill(const Csr &A, Sten &S, hipStream_t s)
    S.dict = dalloc_n<double>((size_t) ns * ST_DICT);
    S.nslices = ns;
    k_sten_fill<<<std::min(ns, SF_GRID), 64, 0, s>>>(A.nrows, ns, S.tab, A.ia, A.ja, A.a, S.mask,
-                                                    S.info, S.codes, S.dict, &S.head->raw);
+                                                    S.info, S.codes, S.dict, &S.head->raw, &S.head->coded);
    HX_LAUNCH_CHECK();
-   HX_HIP(hipMemcpyAsync(&sten_pinned()->raw, &S.head->raw, sizeof(int), hipMemcpyDeviceToHost, s));
+   HX_HIP(hipMemcpyAsync(&sten_pinned()->raw, &S.head->raw, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
 }
 
-int sten_raw_slices() { return sten_pinned()->raw; }
+void sten_counts(Sten &S)
+{
+   S.tab.raw = sten_pinned()->raw;
+   S.tab.coded = sten_pinned()->coded;
+}
 
 void sten_fill_raw(const Csr &A, Sten &S, bool fp32, hipStream_t s)
 {
@@ -858,6 +906,89 @@ __global__ __launch_bounds__(BS) void k_relax_l1_sten(int n, int ns, StenView S,
          const X v0 = w * o.a.a - w * t.a, v1 = w * o.a.b - w * t.b;
          sten_put(uo, row, both, o.b.a + v0 / o.c.a, o.b.b + v1 / o.c.b);
       });
+}
+
+// ---------------------------------------------------------------- step masks of the strength pass
+// One wave a slice, two rows a lane; the values come from the copy, the C/F
+// flags of the neighbours at scalar bases, so a row costs its copy's bytes and
+// 16 written (27-point 200^3: 0.26 ms, where the lists of C neighbours from the
+// CSR entries take 1.4 ms).
+__global__ __launch_bounds__(BS) void k_sten_masks(int n, int ns, StenView S,
+                                                   const double *__restrict__ raw,
+                                                   const double *__restrict__ thr,
+                                                   const int *__restrict__ flg,
+                                                   const int *__restrict__ CF, uint4 *__restrict__ q)
+{
+   __shared__ double sdict[WPB * ST_DICT];
+   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+   double *sd = sdict + wv * ST_DICT;
+   const StenTab T = reinterpret_cast<StenTab>(reinterpret_cast<uintptr_t>(S.tab));
+   const int D = T->D, CW = (D + 3) / 4;
+   const long long lo = D > 1 ? (T->off[1] < 0 ? T->off[1] : 0) : 0;
+   const long long hi = D > 1 ? (T->off[D - 1] > 0 ? T->off[D - 1] : 0) : 0;
+   for (int sl = blockIdx.x * WPB + wv; sl < ns; sl += gridDim.x * WPB) {
+      const int info = __builtin_amdgcn_readfirstlane(S.info[sl]);
+      const int mode = info & 3;
+      const long long f = (long long) sl * ST_ROWS, r = f + 2 * lane;
+      const bool edge = f + lo < 0 || f + ST_ROWS - 1 + hi >= n;
+      const st_uns2 m = *reinterpret_cast<const st_uns2 *>(S.mask + r);
+      const int r0 = (int) min(r, (long long) n - 1), r1 = (int) min(r + 1, (long long) n - 1);
+      const double t0 = thr[r0], t1 = thr[r1];
+      const int f0 = flg[r0], f1 = flg[r1];
+      if (mode == ST_CODES) {
+         __builtin_amdgcn_wave_barrier();
+         for (int i = lane; i < (info >> 8); i += 64) { sd[i] = S.dict[(size_t) sl * ST_DICT + i]; }
+         __builtin_amdgcn_wave_barrier();
+      }
+      const double *rw = raw + (size_t) sl * ST_ROWS * D;
+      uint4 a = {0u, 0u, 0u, 0u}, b = {0u, 0u, 0u, 0u};
+#pragma unroll 1
+      for (int k0 = 0; k0 < D; k0 += 4) {
+         st_uns2 w = {0u, 0u};
+         if (mode == ST_CODES) {
+            w = *reinterpret_cast<const st_uns2 *>(S.codes + ((size_t) sl * CW + (k0 >> 2)) * ST_ROWS + 2 * lane);
+         }
+#pragma unroll
+         for (int u = 0; u < 4; u++) {
+            const int k = k0 + u;
+            if (k == 0 || k >= D) { continue; }   // uniform
+            const Two<double> v =
+               mode == ST_CONST ? sten_value<ST_CONST, double, double>(k, lane, T, &w, sd, rw)
+               : mode == ST_RAW ? sten_value<ST_RAW, double, double>(k, lane, T, &w, sd, rw)
+                                : sten_value<ST_CODES, double, double>(u, lane, T, &w, sd, rw);
+            const long long j = r + T->off[k];
+            int c0, c1;
+            if (edge) {
+               c0 = CF[j < 0 ? 0 : j >= n ? n - 1 : j];
+               c1 = CF[j < -1 ? 0 : j >= n - 1 ? n - 1 : j + 1];
+            } else {
+               c0 = CF[j];
+               c1 = CF[j + 1];
+            }
+            const unsigned bit = 1u << k;
+            auto put = [&](uint4 &z, unsigned mk, double val, double t, int fl, int c) {
+               if (!(mk & bit)) { return; }
+               const bool neg = fl & 1;
+               if (!(fl & 2) && (neg ? !(val <= t) : !(val >= t))) { z.x |= bit; }
+               if (c >= 0) { z.y |= bit; }
+               if (c == -3) { z.z |= bit; }
+               if (neg ? val > 0 : val < 0) { z.w |= bit; }
+            };
+            put(a, m.x, v.a, t0, f0, c0);
+            put(b, m.y, v.b, t1, f1, c1);
+         }
+      }
+      if (r < n) { q[r] = a; }
+      if (r + 1 < n) { q[r + 1] = b; }
+   }
+}
+
+void sten_masks(const Csr &A, const Sten &S, const double *thr, const int *flg, const int *CF, uint4 *q)
+{
+   const StenView v{S.head, S.mask, S.codes, S.info, S.dict};
+   const int nb = (int) std::min<long long>(((long long) S.nslices + WPB - 1) / WPB, 2048);
+   k_sten_masks<<<nb, BS, 0, stream()>>>(A.nrows, S.nslices, v, S.raw, thr, flg, CF, q);
+   HX_LAUNCH_CHECK();
 }
 
 // tables with the runs of a usual grid stencil are unrolled exactly; others

@@ -5,8 +5,10 @@ the fine operator's columns differ from the row by at most 32 offsets: slices
 of 128 rows with no values, with a dictionary of at most 256, or with full
 values.  A V-cycle in FP64 and FP32 must agree bit for bit between the two on
 grids whose slices are cut by lines, planes and the matrix's end, on the
-table sizes with an unrolled kernel (5, 7, 9, 19, 27) and others, at 32 and
-33 offsets, and on rows that are not sorted (both fall back).
+table sizes with an unrolled kernel (5, 7, 9, 19, 27) and others, at 31 and
+33 offsets, and on rows that are not sorted (both fall back).  The fine level's
+interpolation, which the stencil path forms one lane a row, must be the
+general kernels' bits for every threshold, truncation and sign pattern.
 """
 import numpy as np
 import pytest
@@ -14,10 +16,11 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False, special=None):
+def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False, positive=0.0):
     """Rows diagonal first, then ascending, from (dx, dy, dz) offsets in
     symmetric pairs; values 'const', 'few' (64 distinct couplings) or 'all'
-    (every coupling its own); missing: share of the pairs left out."""
+    (every coupling its own); missing: share of the pairs left out; positive:
+    share of small couplings of the diagonal's sign."""
     import scipy.sparse as sp
     rng = np.random.default_rng(seed)
     n = nx * ny * nz
@@ -33,12 +36,13 @@ def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False,
         j = i + (dz * ny + dy) * nx + dx
         v = {"const": np.ones(len(i)), "few": 0.5 + rng.integers(0, 64, len(i)) / 64.0,
              "all": 0.5 + rng.random(len(i))}[values]
+        v = np.where(rng.random(len(i)) < positive, -0.3 * v, v)
         rows += [i, j]
         cols += [j, i]
         vals += [-v, -v]
     off = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))), shape=(n, n))
     off.sort_indices()
-    diag = 1e-2 - np.asarray(off.sum(axis=1)).ravel()
+    diag = 1e-2 + np.asarray(abs(off).sum(axis=1)).ravel()
     if values == "const":
         diag[:] = diag.max()
     ia = np.zeros(n + 1, np.int32)
@@ -125,3 +129,39 @@ def test_product_with_dot_matches_the_csr_kernels(hx, oracle):
     assert out[0][0] == out[1][0]
     np.testing.assert_allclose(out[1][1], out[0][1], rtol=1e-9)
     np.testing.assert_allclose(out[1][2], out[0][2], rtol=1e-8, atol=1e-12 * np.abs(out[0][2]).max())
+
+
+INTERP = {
+    "27_const": (17, 19, 23, box(), "const", {}),
+    "27_few": (21, 16, 17, box(), "few", {}),
+    "27_all_signs": (19, 17, 16, box(), "all", {"positive": 0.2}),
+    "27_missing": (19, 17, 16, box(), "few", {"missing": 0.25}),
+    "27_thin": (2, 61, 47, box(), "few", {}),
+    "19_signs": (18, 15, 19, P19, "few", {"positive": 0.1}),
+    "9_all": (131, 67, 1, P9, "all", {}),
+    "7_const": (20, 21, 22, P7, "const", {}),
+    "7_signs_missing": (33, 13, 14, P7, "few", {"missing": 0.1, "positive": 0.1}),
+    "31_all": (5003, 1, 1, P31, "all", {"missing": 0.3}),
+}
+
+
+@pytest.mark.parametrize("options", [
+    {}, {"strong_threshold": 0.6}, {"strong_threshold": 0.95, "max_row_sum": 1.0},
+    {"strong_threshold": 0.01, "P_max_elmts": 32}, {"P_max_elmts": 1, "trunc_factor": 0.3},
+    {"coarsen_type": 10, "trunc_factor": 0.1}], ids=lambda o: ",".join(f"{k}={v}" for k, v in o.items()) or "default")
+@pytest.mark.parametrize("name", sorted(INTERP))
+def test_interpolation_bits_equal_the_general_kernels(hx, name, options):
+    nx, ny, nz, offsets, values, more = INTERP[name]
+    print("[gpu-stencil] P", name, options, flush=True)
+    A = hx.ParCSRMatrix.from_csr(*grid_matrix(nx, ny, nz, offsets, values, **more))
+    got = []
+    for fmt in (0, 1):
+        amg = hx.BoomerAMG(solve_format=fmt, max_levels=2, **options)
+        amg.setup(A)
+        got.append((amg.level_cf(0), amg.level_matrix(0, "P")))
+        amg.destroy()
+    (cf0, P0), (cf1, P1) = got
+    assert np.array_equal(cf0, cf1)
+    assert np.array_equal(P0.ia, P1.ia) and np.array_equal(P0.ja, P1.ja)
+    bad = np.nonzero(P0.a.view(np.int64) != P1.a.view(np.int64))[0]
+    assert bad.size == 0, f"{bad.size} of {P0.nnz} weights differ, first at {bad[:5]}"

@@ -23,7 +23,8 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libhypre_mi355x.so")
 ARCH = os.environ.get("HYPRE_MI355X_ARCH", "gfx950")
 
-SOURCES = ["hx_runtime.hip", "hx_solve.hip", "hx_stencil.hip", "hx_setup.hip", "hx_amg.hip", "hx_ij.hip",
+SOURCES = ["hx_runtime.hip", "hx_solve.hip", "hx_stencil.hip", "hx_setup.hip", "hx_amg.hip",
+           "hx_ij.hip", "hx_ijasm.hip",
            "hx_mlp.hip", "hx_hmis.hip", "hx_agg.hip", "hx_noalloc.hip", "hx_stats.hip"]
 
 CFLAGS = [

@@ -34,7 +34,10 @@ struct hypre_IJMatrix_struct
    std::vector<int>    st_row, st_col;
    std::vector<double> st_val;
    std::vector<char>   st_op;
-   // assembled host copy (for updates after assembly)
+   // operations already on the device, before the staged ones
+   std::vector<IjChunk> chunks;
+   // assembled host copy (for updates after assembly), fetched when needed
+   bool                h_valid = false;
    std::vector<int>    h_ia, h_ja;
    std::vector<double> h_a;
    hypre_ParCSRMatrix_struct *par = nullptr;
@@ -213,6 +216,44 @@ static void ij_assemble_host(hypre_IJMatrix_struct *m)
    m->h_ia.swap(ia);
    m->h_ja.swap(ja);
    m->h_a.swap(a);
+   m->h_valid = true;
+}
+
+// the host copy of an assembled matrix
+static void ij_host(hypre_IJMatrix_struct *m)
+{
+   if (m->h_valid || !m->par) { return; }
+   csr_to_host(m->par->A, m->h_ia, m->h_ja, m->h_a);
+   m->h_valid = true;
+}
+
+// Operations of a call, or of a whole assembly, from which the device assembles.
+// Below, the host is done in the time that the uploads, launches and read-backs
+// take (0.3 to 0.5 ms): 16000 operations 0.19 ms on the host, 32000 0.47, 64000
+// 0.85 against 0.48 on the device.
+constexpr size_t IJ_DEVICE_MIN = 32768;
+
+static void ij_clear_staged(hypre_IJMatrix_struct *m)
+{
+   m->st_row.clear(); m->st_col.clear(); m->st_val.clear(); m->st_op.clear();
+   m->st_row.shrink_to_fit(); m->st_col.shrink_to_fit(); m->st_val.shrink_to_fit(); m->st_op.shrink_to_fit();
+}
+
+// the operations staged on the host become a chunk
+static void ij_flush_staged(hypre_IJMatrix_struct *m)
+{
+   if (m->st_row.empty()) { return; }
+   if (m->st_row.size() > (size_t) INT_MAX) { fail(HYPRE_ERROR_MEMORY, "too many operations for one assembly"); }
+   m->chunks.reserve(m->chunks.size() + 1);
+   m->chunks.push_back(ij_chunk((int) m->st_row.size(), (long long) m->st_row.size(), m->st_row.data(), nullptr,
+                                m->st_col.data(), m->st_val.data(), m->st_op.data(), 0));
+   ij_clear_staged(m);
+}
+
+static void ij_free_chunks(hypre_IJMatrix_struct *m)
+{
+   for (IjChunk &c : m->chunks) { c.free_all(); }
+   m->chunks.clear();
 }
 
 template <class T>
@@ -243,6 +284,18 @@ static void ij_stage(hypre_IJMatrix_struct *m, HYPRE_Int nrows, HYPRE_Int *ncols
    if (!cols) { g_error_arg = 5; fail(HYPRE_ERROR_ARG, "NULL cols"); }
    if (!values) { g_error_arg = 6; fail(HYPRE_ERROR_ARG, "NULL values"); }
    std::vector<int> nc = fetch_input<int>(ncols, (size_t) nrows, m->memloc);
+   if (!m->assembled && (int) m->chunks.size() < IJ_CHUNKS - 2) {
+      size_t ops = 0;
+      for (int i = 0; i < nrows; i++) { ops += (size_t) nc[(size_t) i]; }
+      if (ops >= IJ_DEVICE_MIN && ops <= (size_t) INT_MAX) {
+         // a large call goes to the device as it is
+         ensure_init();
+         ij_flush_staged(m);
+         m->chunks.reserve(m->chunks.size() + 1);
+         m->chunks.push_back(ij_chunk(nrows, (long long) ops, rows, ncols, cols, values, nullptr, op));
+         return;
+      }
+   }
    std::vector<int> rw = fetch_input<int>(rows, (size_t) nrows, m->memloc);
    size_t total = 0;
    for (int i = 0; i < nrows; i++) { total += (size_t) nc[(size_t) i]; }
@@ -250,6 +303,7 @@ static void ij_stage(hypre_IJMatrix_struct *m, HYPRE_Int nrows, HYPRE_Int *ncols
    std::vector<double> vl = fetch_input<double>(values, total, m->memloc);
    if (m->assembled) {
       // update existing entries of the assembled matrix (hypre: entries must exist)
+      ij_host(m);
       size_t k = 0;
       for (int i = 0; i < nrows; i++) {
          const int r = rw[(size_t) i] - m->ilower;
@@ -310,6 +364,7 @@ HYPRE_Int HYPRE_IJMatrixDestroy(HYPRE_IJMatrix m)
 {
    return guard([&] {
       if (!m) { return; }
+      ij_free_chunks(m);
       if (m->par) { m->par->A.free_all(); delete m->par; }
       delete m;
    });
@@ -354,10 +409,24 @@ HYPRE_Int HYPRE_IJMatrixAssemble(HYPRE_IJMatrix m)
       if (!m) { g_error_arg = 1; fail(HYPRE_ERROR_ARG, "NULL IJ matrix"); }
       const int nrows = m->iupper - m->ilower + 1;
       const int ncols = m->jupper - m->jlower + 1;
+      if (!m->chunks.empty() || m->st_row.size() >= IJ_DEVICE_MIN) {
+         ij_flush_staged(m);
+         Csr A;
+         if (!ij_assemble_device(m->chunks, m->ilower, nrows, m->jlower, ncols, m->direct_insert, A)) {
+            fail(HYPRE_ERROR_GENERIC, "column index outside [jlower, jupper]");
+         }
+         ij_free_chunks(m);
+         if (m->par) { m->par->A.free_all(); delete m->par; }
+         m->par = new hypre_ParCSRMatrix_struct();
+         m->par->A = A;
+         m->h_valid = false;
+         m->modified = false;
+         m->assembled = true;
+         return;
+      }
       if (!(m->assembled && m->modified)) { ij_assemble_host(m); }
       m->modified = false;
-      m->st_row.clear(); m->st_col.clear(); m->st_val.clear(); m->st_op.clear();
-      m->st_row.shrink_to_fit(); m->st_col.shrink_to_fit(); m->st_val.shrink_to_fit(); m->st_op.shrink_to_fit();
+      ij_clear_staged(m);
       if (m->par) { m->par->A.free_all(); delete m->par; m->par = nullptr; }
       m->par = par_from_host(nrows, ncols, m->h_ia.data(), m->h_ja.data(), m->h_a.data());
       m->assembled = true;
@@ -429,6 +498,7 @@ HYPRE_Int HYPRE_IJMatrixGetRowCounts(HYPRE_IJMatrix m, HYPRE_Int nrows, HYPRE_Bi
 {
    return guard([&] {
       if (!m->assembled) { fail(HYPRE_ERROR_GENERIC, "IJ matrix not assembled"); }
+      ij_host(m);
       for (int i = 0; i < nrows; i++) {
          int r = rows[i] - m->ilower;
          ncols[i] = m->h_ia[(size_t) r + 1] - m->h_ia[(size_t) r];
@@ -441,6 +511,7 @@ HYPRE_Int HYPRE_IJMatrixGetValues(HYPRE_IJMatrix m, HYPRE_Int nrows, HYPRE_Int *
 {
    return guard([&] {
       if (!m->assembled) { fail(HYPRE_ERROR_GENERIC, "IJ matrix not assembled"); }
+      ij_host(m);
       size_t k = 0;
       for (int i = 0; i < nrows; i++) {
          int r = rows[i] - m->ilower;
@@ -566,6 +637,7 @@ HYPRE_Int HYPRE_IJMatrixPrint(HYPRE_IJMatrix m, const char *filename)
    return guard([&] {
       if (!m || m->object_type != HYPRE_PARCSR) { g_error_arg = 1; fail(HYPRE_ERROR_ARG, "bad IJ matrix"); }
       if (!m->assembled) { fail(HYPRE_ERROR_GENERIC, "IJ matrix not assembled"); }
+      ij_host(m);
       const std::string path = rank_file(filename, "");
       FileCloser fc{fopen(path.c_str(), "w")};
       if (!fc.fp) { g_error_arg = 2; fail(HYPRE_ERROR_ARG, "cannot open " + path); }
@@ -654,6 +726,7 @@ HYPRE_Int HYPRE_IJMatrixPrintBinary(HYPRE_IJMatrix m, const char *filename)
    return guard([&] {
       if (!m || m->object_type != HYPRE_PARCSR) { g_error_arg = 1; fail(HYPRE_ERROR_ARG, "bad IJ matrix"); }
       if (!m->assembled) { fail(HYPRE_ERROR_GENERIC, "IJ matrix not assembled"); }
+      ij_host(m);
       const std::string path = rank_file(filename, ".bin");
       FileCloser fc{fopen(path.c_str(), "wb")};
       if (!fc.fp) { fail(HYPRE_ERROR_GENERIC, "Could not open output file " + path); }

@@ -238,6 +238,26 @@ int sten_spmv(const Csr &A, X alpha, const X *x, X beta, const X *b, X *y, doubl
 template <typename V, typename X>
 void sten_relax_l1(const Csr &A, const X *f, const X *u, const X *l1, X w, X *uo);
 
+// The operations of an IJ matrix in call order, as assembled on the device:
+// one call's arrays, or single staged operations (ncols nullptr, ops set)
+struct IjChunk
+{
+   int        nseg = 0;
+   long long  nops = 0;
+   int       *rows = nullptr, *ncols = nullptr, *cols = nullptr;
+   double    *vals = nullptr;
+   char      *ops = nullptr;
+   char       op = 0;             // 0 set, 1 add, for all (ops nullptr)
+   void       free_all();
+};
+constexpr int IJ_CHUNKS = 32;     // most chunks of one assembly
+// uploads (waits: the arrays may be reused at once)
+IjChunk ij_chunk(int nseg, long long nops, const int *rows, const int *ncols, const int *cols,
+                 const double *vals, const char *ops, char op);
+// A from the chunks; false when some column lies outside [jlower, jlower + ncols)
+bool ij_assemble_device(const std::vector<IjChunk> &chunks, int ilower, int nrows, int jlower, int ncols,
+                        bool swap_diag, Csr &A);
+
 void csr_copy(const Csr &src, Csr &dst);
 void csr_to_host(const Csr &A, std::vector<int> &ia, std::vector<int> &ja, std::vector<double> &a);
 void csr_from_host(Csr &A, int n, int ncols, const int *ia, const int *ja, const double *a);

@@ -16,7 +16,11 @@
 // the same order).
 #include "hx_internal.h"
 
+#include <sys/mman.h>
+
 #include <algorithm>
+#include <cstdlib>
+#include <new>
 #include <vector>
 
 namespace hx {
@@ -25,31 +29,40 @@ namespace {
 
 constexpr int kC = 1, kF = -1, kZ = -2, kSF = -3;
 
+// a point's list links, measure and state in 16 bytes: the pass visits points in
+// no order that a cache could follow, and each visit needs all four
+struct Point
+{
+   int next, prev, measure, cf;
+};
+
 struct MeasureBuckets
 {
    std::vector<int> head, tail;   // per measure value
-   std::vector<int> next, prev;   // per point
+   Point *pt;
    int top = 0;                   // no bucket above `top` holds a point
 
-   explicit MeasureBuckets(int n) : next(n, -1), prev(n, -1) {}
+   explicit MeasureBuckets(Point *p) : head(64, -1), tail(64, -1), pt(p) {}
 
    void push(int m, int i)
    {
       if (m >= (int) head.size()) {
-         head.resize(m + 1, -1);
-         tail.resize(m + 1, -1);
+         head.resize(2 * m + 1, -1);
+         tail.resize(2 * m + 1, -1);
       }
-      next[i] = -1;
-      prev[i] = tail[m];
-      if (tail[m] >= 0) { next[tail[m]] = i; } else { head[m] = i; }
+      const int t = tail[m];
+      pt[i].next = -1;
+      pt[i].prev = t;
+      if (t >= 0) { pt[t].next = i; } else { head[m] = i; }
       tail[m] = i;
       top = std::max(top, m);
    }
 
    void erase(int m, int i)
    {
-      if (prev[i] >= 0) { next[prev[i]] = next[i]; } else { head[m] = next[i]; }
-      if (next[i] >= 0) { prev[next[i]] = prev[i]; } else { tail[m] = prev[i]; }
+      const int nx = pt[i].next, pv = pt[i].prev;
+      if (pv >= 0) { pt[pv].next = nx; } else { head[m] = nx; }
+      if (nx >= 0) { pt[nx].prev = pv; } else { tail[m] = pv; }
    }
 
    // first point of the largest non-empty measure (-1 when all are empty)
@@ -60,93 +73,123 @@ struct MeasureBuckets
    }
 };
 
+// memory that is not cleared first and comes in large pages where it can
+template <class T>
+struct Raw
+{
+   T *p;
+   explicit Raw(size_t n)
+   {
+      const size_t page = size_t(2) << 20, bytes = (std::max<size_t>(n, 1) * sizeof(T) + page - 1) / page * page;
+      p = static_cast<T *>(std::aligned_alloc(page, bytes));
+      if (!p) { throw std::bad_alloc(); }
+      (void) madvise(p, bytes, MADV_HUGEPAGE);
+   }
+   ~Raw() { std::free(p); }
+   Raw(const Raw &) = delete;
+   Raw &operator=(const Raw &) = delete;
+   T &operator[](size_t i) { return p[i]; }
+};
+
 } // namespace
 
-// par_coarsen.c:1060-1391 for one rank, measure_type 0, cut_factor 0
-void rs_first_pass_host(int n, const int *Si, const int *Sj, int *CF)
+// par_coarsen.c:1060-1391 for one rank, measure_type 0, cut_factor 0.
+// STi, STj: S^T, each row ascending.  The pass follows S and S^T from point to
+// point and each step needs the one before, so it stays on one host thread; a
+// point is one 16-byte record, and rows that come next are asked for ahead.
+static void rs_first_pass(int n, const int *Si, const int *Sj, const int *STi, const int *STj, int *CF)
 {
-   const int nnz = Si[n];
-   // S^T (stable counting sort): the points that depend on each point
-   std::vector<int> STi(n + 1, 0), STj(std::max(nnz, 1));
-   for (int k = 0; k < nnz; k++) { STi[Sj[k] + 1]++; }
-   for (int i = 0; i < n; i++) { STi[i + 1] += STi[i]; }
-   {
-      std::vector<int> pos(STi.begin(), STi.end() - 1);
-      for (int i = 0; i < n; i++) {
-         for (int k = Si[i]; k < Si[i + 1]; k++) { STj[pos[Sj[k]]++] = i; }
-      }
-   }
-   std::vector<int> measure(n);
-   for (int i = 0; i < n; i++) { measure[i] = STi[i + 1] - STi[i]; }
-
+   Raw<Point> pts((size_t) n);
+   Point *pt = pts.p;
    int num_left = 0;
    for (int j = 0; j < n; j++) {
       if (Si[j + 1] == Si[j]) {
-         CF[j] = kSF;
-         measure[j] = 0;
+         pt[j] = Point{-1, -1, 0, kSF};
       } else {
-         CF[j] = 0;
+         pt[j] = Point{-1, -1, STi[j + 1] - STi[j], 0};
          num_left++;
       }
    }
-   MeasureBuckets B(n);
+   MeasureBuckets B(pt);
    // points nobody depends on become Z; their neighbours' measures grow
    for (int j = 0; j < n; j++) {
-      if (CF[j] == kSF) { continue; }
-      if (measure[j] > 0) {
-         B.push(measure[j], j);
+      if (pt[j].cf == kSF) { continue; }
+      if (pt[j].measure > 0) {
+         B.push(pt[j].measure, j);
          continue;
       }
-      CF[j] = kZ;
+      pt[j].cf = kZ;
       for (int k = Si[j]; k < Si[j + 1]; k++) {
          const int nb = Sj[k];
-         if (CF[nb] == kSF) { continue; }
+         if (pt[nb].cf == kSF) { continue; }
          if (nb < j) {
-            if (measure[nb] > 0) { B.erase(measure[nb], nb); }
-            B.push(++measure[nb], nb);
+            if (pt[nb].measure > 0) { B.erase(pt[nb].measure, nb); }
+            B.push(++pt[nb].measure, nb);
          } else {
-            ++measure[nb];
+            ++pt[nb].measure;
          }
       }
       --num_left;
    }
    // a point that becomes F raises the measures of its undecided influences
    auto raise_influences = [&](int p) {
-      for (int k = Si[p]; k < Si[p + 1]; k++) {
+      const int e = Si[p + 1];
+      for (int k = Si[p]; k < e; k++) {
          const int q = Sj[k];
-         if (CF[q] != 0) { continue; }
-         B.erase(measure[q], q);
-         B.push(++measure[q], q);
+         if (k + 8 < e) { __builtin_prefetch(pt + Sj[k + 8], 1); }
+         if (pt[q].cf != 0) { continue; }
+         B.erase(pt[q].measure, q);
+         B.push(++pt[q].measure, q);
       }
    };
    while (num_left > 0) {
       const int c = B.front();
       if (c < 0) { fail(HYPRE_ERROR_GENERIC, "HMIS first pass: no undecided point left"); }
-      CF[c] = kC;
-      B.erase(measure[c], c);
-      measure[c] = 0;
+      pt[c].cf = kC;
+      B.erase(pt[c].measure, c);
+      pt[c].measure = 0;
       --num_left;
-      for (int k = STi[c]; k < STi[c + 1]; k++) {
+      const int e = STi[c + 1];
+      for (int k = STi[c]; k < e; k++) { __builtin_prefetch(Sj + Si[STj[k]]); }
+      for (int k = STi[c]; k < e; k++) {
          const int nb = STj[k];
-         if (CF[nb] != 0) { continue; }
-         CF[nb] = kF;
-         B.erase(measure[nb], nb);
+         if (pt[nb].cf != 0) { continue; }
+         pt[nb].cf = kF;
+         B.erase(pt[nb].measure, nb);
          --num_left;
          raise_influences(nb);
       }
       for (int k = Si[c]; k < Si[c + 1]; k++) {
          const int nb = Sj[k];
-         if (CF[nb] != 0) { continue; }
-         B.erase(measure[nb], nb);
-         if (--measure[nb] > 0) {
-            B.push(measure[nb], nb);
+         if (pt[nb].cf != 0) { continue; }
+         B.erase(pt[nb].measure, nb);
+         if (--pt[nb].measure > 0) {
+            B.push(pt[nb].measure, nb);
          } else {
-            CF[nb] = kF;
+            pt[nb].cf = kF;
             --num_left;
             raise_influences(nb);
          }
       }
    }
+   for (int j = 0; j < n; j++) { CF[j] = pt[j].cf; }
+}
+
+void rs_first_pass_host(int n, const int *Si, const int *Sj, int *CF)
+{
+   const int nnz = Si[n];
+   // S^T (stable counting sort): the points that depend on each point
+   std::vector<int> STi((size_t) n + 1, 0);
+   Raw<int> STj((size_t) nnz);
+   for (int k = 0; k < nnz; k++) { STi[(size_t) Sj[k] + 1]++; }
+   for (int i = 0; i < n; i++) { STi[i + 1] += STi[i]; }
+   {
+      std::vector<int> pos(STi.begin(), STi.end() - 1);
+      for (int i = 0; i < n; i++) {
+         for (int k = Si[i]; k < Si[i + 1]; k++) { STj[(size_t) pos[Sj[k]]++] = i; }
+      }
+   }
+   rs_first_pass(n, Si, Sj, STi.data(), STj.p, CF);
 }
 
 int hmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_keep_dev,
@@ -155,11 +198,24 @@ int hmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_ke
    const int n = S.nrows;
    if (n == 0) { return 0; }
    TimedLaunch tl("setup_hmis_first_pass", 0.0);
-   std::vector<int> ia(n + 1), ja(std::max<long long>(S.nnz, 1)), cf(n);
-   d2h(ia.data(), S.ia, sizeof(int) * ((size_t) n + 1));
-   if (S.nnz > 0) { d2h(ja.data(), S.ja, sizeof(int) * (size_t) S.nnz); }
-   rs_first_pass_host(n, ia.data(), ja.data(), cf.data());
-   h2d(CF, cf.data(), sizeof(int) * (size_t) n);
+   // S^T comes from the device, where it takes 0.6 ms (level 0 of 27-point
+   // 64^3): on the host it was nearly half of the pass, and clearing vectors for
+   // the copies a part of the rest (all levels of 64^3: 31 to 37 ms -> 22.5)
+   Csr ST;
+   transpose(S, ST, false);
+   Raw<int> ia((size_t) n + 1), ja((size_t) S.nnz), tia((size_t) n + 1), tja((size_t) S.nnz), cf((size_t) n);
+   try {
+      d2h(ia.p, S.ia, sizeof(int) * ((size_t) n + 1));
+      d2h(tia.p, ST.ia, sizeof(int) * ((size_t) n + 1));
+      d2h(ja.p, S.ja, sizeof(int) * (size_t) S.nnz);
+      d2h(tja.p, ST.ja, sizeof(int) * (size_t) S.nnz);
+   } catch (...) {
+      ST.free_all();
+      throw;
+   }
+   ST.free_all();
+   rs_first_pass(n, ia.p, ja.p, tia.p, tja.p, cf.p);
+   h2d(CF, cf.p, sizeof(int) * (size_t) n);
    return pmis(S, measure_in_dev, CF, measure_keep_dev, st_count, 1);
 }
 

@@ -3890,6 +3890,8 @@ __global__ __launch_bounds__(256) void k_col_count_h(long long nnz, const int *_
    }
 }
 
+// VALUES false: the pattern alone (a, Ra unused)
+template <bool VALUES>
 __global__ __launch_bounds__(256) void k_t_fill_h(int n, const int *__restrict__ ia,
                                                   const int *__restrict__ ja,
                                                   const double *__restrict__ a,
@@ -3942,13 +3944,13 @@ __global__ __launch_bounds__(256) void k_t_fill_h(int n, const int *__restrict__
             const int k = s + t;
             const int pos = (slot[t] >= 0) ? hval[slot[t]] + li[t] : atomicAdd(&fillp[ja[k]], 1);
             Rj[pos] = i;
-            Ra[pos] = a[k];
+            if (VALUES) { Ra[pos] = a[k]; }
          }
       }
       for (int k = s + TF_E; k < e; k++) {
          const int pos = atomicAdd(&fillp[ja[k]], 1);
          Rj[pos] = i;
-         Ra[pos] = a[k];
+         if (VALUES) { Ra[pos] = a[k]; }
       }
       __syncthreads();
    }
@@ -3959,6 +3961,7 @@ __global__ __launch_bounds__(256) void k_t_fill_h(int n, const int *__restrict__
 // stage are sorted by insertion in lane 0.
 constexpr int TS_MAX = 512;
 
+template <bool VALUES>
 __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__ Ria,
                                                  int *__restrict__ Rj, double *__restrict__ Ra)
 {
@@ -3974,7 +3977,7 @@ __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__
       e = Ria[r + 1];
       if (e - b <= WAVE && lane < e - b) {
          key = Rj[b + lane];
-         val = Ra[b + lane];
+         if (VALUES) { val = Ra[b + lane]; }
       }
    };
    if (blockIdx.x < nc) { fetch(blockIdx.x); }
@@ -3991,7 +3994,7 @@ __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__
             int rank = 0;
             for (int m = 0; m < L; m++) { rank += (sk[m] < ckey) ? 1 : 0; }
             Rj[cb + rank] = ckey;
-            Ra[cb + rank] = cval;
+            if (VALUES) { Ra[cb + rank] = cval; }
          }
          wave_sync();
          continue;
@@ -4000,22 +4003,22 @@ __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__
          if (lane == 0) {
             for (int k = cb + 1; k < ce; k++) {
                const int key = Rj[k];
-               const double v = Ra[k];
+               const double v = VALUES ? Ra[k] : 0.0;
                int m = k - 1;
                while (m >= cb && Rj[m] > key) {
                   Rj[m + 1] = Rj[m];
-                  Ra[m + 1] = Ra[m];
+                  if (VALUES) { Ra[m + 1] = Ra[m]; }
                   m--;
                }
                Rj[m + 1] = key;
-               Ra[m + 1] = v;
+               if (VALUES) { Ra[m + 1] = v; }
             }
          }
          continue;
       }
       for (int k = lane; k < L; k += WAVE) {
          sk[k] = Rj[cb + k];
-         sv[k] = Ra[cb + k];
+         if (VALUES) { sv[k] = Ra[cb + k]; }
       }
       wave_sync();
       for (int k = lane; k < L; k += WAVE) {
@@ -4023,13 +4026,13 @@ __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__
          int rank = 0;
          for (int m = 0; m < L; m++) { rank += (sk[m] < key) ? 1 : 0; }
          Rj[cb + rank] = key;
-         Ra[cb + rank] = sv[k];
+         if (VALUES) { Ra[cb + rank] = sv[k]; }
       }
       wave_sync();
    }
 }
 
-void transpose(const Csr &P, Csr &R)
+void transpose(const Csr &P, Csr &R, bool values)
 {
    int n = P.nrows, nc = P.ncols;
    TimedLaunch tl("setup_transpose", 0.0);
@@ -4038,7 +4041,7 @@ void transpose(const Csr &P, Csr &R)
    R.nnz = P.nnz;
    R.ia = dalloc_n<int>((size_t) nc + 1);
    R.ja = dalloc_n<int>((size_t) std::max<long long>(P.nnz, 1));
-   R.a = dalloc_n<double>((size_t) std::max<long long>(P.nnz, 1));
+   R.a = values ? dalloc_n<double>((size_t) std::max<long long>(P.nnz, 1)) : nullptr;
    R.a32 = nullptr;
    dzero(R.ia, sizeof(int) * ((size_t) nc + 1));
    const long long nch = (P.nnz + 256LL * TC_U - 1) / (256LL * TC_U);
@@ -4049,8 +4052,13 @@ void transpose(const Csr &P, Csr &R)
    int *fillp = dalloc_n<int>((size_t) nc + 1);
    d2d(fillp, R.ia, sizeof(int) * ((size_t) nc + 1));
    int nb = std::max(1, std::min((n + 255) / 256, 8192));
-   k_t_fill_h<<<nb, 256, 0, stream()>>>(n, P.ia, P.ja, P.a, fillp, R.ja, R.a);
-   k_t_sort<<<launch_blocks(nc), WAVE, 0, stream()>>>(nc, R.ia, R.ja, R.a);
+   if (values) {
+      k_t_fill_h<true><<<nb, 256, 0, stream()>>>(n, P.ia, P.ja, P.a, fillp, R.ja, R.a);
+      k_t_sort<true><<<launch_blocks(nc), WAVE, 0, stream()>>>(nc, R.ia, R.ja, R.a);
+   } else {
+      k_t_fill_h<false><<<nb, 256, 0, stream()>>>(n, P.ia, P.ja, nullptr, fillp, R.ja, nullptr);
+      k_t_sort<false><<<launch_blocks(nc), WAVE, 0, stream()>>>(nc, R.ia, R.ja, nullptr);
+   }
    HX_LAUNCH_CHECK();
    dfree(fillp);
 }

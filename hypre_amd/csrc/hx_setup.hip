@@ -246,7 +246,7 @@ static int max_row_len(const Csr &A)
 constexpr int RS_SW = 1024;
 constexpr int RS_WPB = 4;
 
-__global__ __launch_bounds__(RS_WPB * WAVE) void k_row_stats(int n, const int *__restrict__ ia,
+__global__ __launch_bounds__(RS_WPB * WAVE) void k_row_stats(int n, int gr, const int *__restrict__ ia,
                                                                const double *__restrict__ a,
                                                                double theta, double mrs,
                                                                double *__restrict__ thr,
@@ -261,12 +261,12 @@ __global__ __launch_bounds__(RS_WPB * WAVE) void k_row_stats(int n, const int *_
    const int blk = xcd_blk(blockIdx.x, nb);
    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
    double *sb = sb_all + wv * RS_SW;
-   const int ng = (n + WAVE - 1) / WAVE;
+   const int ng = (n + gr - 1) / gr;
    const int gpb = (ng + nb - 1) / nb;
    const int g0 = blk * gpb, g1 = min(ng, g0 + gpb);
    for (int g = g0 + wv; g < g1; g += RS_WPB) {
-      const int r0 = g * WAVE;
-      const int nr = min(WAVE, n - r0);
+      const int r0 = g * gr;
+      const int nr = min(gr, n - r0);
       int rs = 0, re = 0;
       if (lane < nr) {
          rs = ia[r0 + lane];
@@ -377,11 +377,21 @@ __global__ void k_strength_recount(int n, const int *__restrict__ ia, const doub
 // also the number of rows in which each column is strong (the columns of
 // S^T), aggregated per block in an LDS table over SF_ROWS consecutive rows.
 constexpr int SF_ROWS = 256;
+
+// rows per block: SF_ROWS, fewer where that leaves most CUs without a block (a
+// level of 970 rows had four, each taking eight rows at a time: 50 us, 9 now),
+// but at least one row for each of the block's groups of K lanes
+static int strength_rows(int n, int K)
+{
+   int rpb = SF_ROWS;
+   while (rpb > 256 / K && (n + rpb - 1) / rpb < 512) { rpb >>= 1; }
+   return rpb;
+}
 constexpr int SF_SLOTS = 4096;
 constexpr int SF_U = 4;
 
 template <int K, bool RUNS>
-__global__ __launch_bounds__(256) void k_strength_fill(int n, const int *__restrict__ ia,
+__global__ __launch_bounds__(256) void k_strength_fill(int n, int rpb, const int *__restrict__ ia,
                                                        const int *__restrict__ ja,
                                                        const double *__restrict__ a,
                                                        const double *__restrict__ thr,
@@ -400,8 +410,8 @@ __global__ __launch_bounds__(256) void k_strength_fill(int n, const int *__restr
       for (int s = threadIdx.x; s < SF_SLOTS; s += 256) { hkey[s] = -1; hcnt[s] = 0; }
       __syncthreads();
    }
-   const long long r_begin = (long long) blockIdx.x * SF_ROWS;
-   const long long r_end = min((long long) n, r_begin + SF_ROWS);
+   const long long r_begin = (long long) blockIdx.x * rpb;
+   const long long r_end = min((long long) n, r_begin + rpb);
    // a row's own operands are loaded one iteration ahead, while the rows
    // before it run
    int n_s = 0, n_e = 0, n_fl = 2, n_o = 0;
@@ -502,11 +512,17 @@ void create_s(const Csr &A, double theta, double max_row_sum, Csr &S, int *st_co
    int *flg = flg_out ? flg_out : dalloc_n<int>((size_t) std::max(n, 1));
    if (st_count) { dzero(st_count, sizeof(int) * (size_t) std::max(n, 1)); }
    if (n > 0) {
-      const long long ng = ((long long) n + WAVE - 1) / WAVE;
+      // rows per wave: 64, fewer on small levels down to about 128 entries, as
+      // the products do (a wave of 64 rows of 140 entries runs nine windows
+      // one after the other): all levels of 7-point 30^3 149 -> 70 us, of a
+      // 7-point problem of 1.67 M rows 478 -> 238
+      int gr = WAVE;
+      while (gr > 4 && (double) A.nnz / n * gr > 128.0 && (n + gr - 1) / gr < 4096) { gr >>= 1; }
+      const long long ng = ((long long) n + gr - 1) / gr;
       long long nbs = std::min<long long>((ng + RS_WPB - 1) / RS_WPB, 8192);
       if (nbs >= 64) { nbs = (nbs + 7) / 8 * 8; }
       k_row_stats<<<(int) std::max<long long>(nbs, 1), RS_WPB * WAVE, 0, stream()>>>(
-          n, A.ia, A.a, theta, max_row_sum, thr, flg, S.ia, l1, l1_zero);
+          n, gr, A.ia, A.a, theta, max_row_sum, thr, flg, S.ia, l1, l1_zero);
       HX_LAUNCH_CHECK();
       const int KR = lanes_per_row_light(A.nnz, n);
       const int nb = (int) std::max<long long>(1, std::min<long long>(((long long) n * KR + 255) / 256, 16384));
@@ -519,14 +535,15 @@ void create_s(const Csr &A, double theta, double max_row_sum, Csr &S, int *st_co
    S.nnz = exclusive_scan(S.ia, S.ia, n);
    S.ja = dalloc_n<int>((size_t) std::max<long long>(S.nnz, 1));
    if (n > 0) {
-      const int nbf = (int) (((long long) n + SF_ROWS - 1) / SF_ROWS);
+      const int rpb = strength_rows(n, K);
+      const int nbf = (int) (((long long) n + rpb - 1) / rpb);
       dispatch_k(K, [&](auto kc) {
          if (column_runs) {
             k_strength_fill<decltype(kc)::value, true><<<nbf, 256, 0, stream()>>>(
-               n, A.ia, A.ja, A.a, thr, flg, S.ia, S.ja, st_count);
+               n, rpb, A.ia, A.ja, A.a, thr, flg, S.ia, S.ja, st_count);
          } else {
             k_strength_fill<decltype(kc)::value, false><<<nbf, 256, 0, stream()>>>(
-               n, A.ia, A.ja, A.a, thr, flg, S.ia, S.ja, st_count);
+               n, rpb, A.ia, A.ja, A.a, thr, flg, S.ia, S.ja, st_count);
          }
       });
       HX_LAUNCH_CHECK();
@@ -614,7 +631,7 @@ __global__ void k_c_lists(int n, const int *__restrict__ ia, const int *__restri
 // entries are those the threshold marks, in A order, i.e. S order, and both
 // lists are compacted in storage order by ballots over the row's lanes.
 template <int K>
-__global__ __launch_bounds__(256) void k_c_lists_t(int n, const int *__restrict__ ia,
+__global__ __launch_bounds__(256) void k_c_lists_t(int n, int rpb, const int *__restrict__ ia,
                                                    const int *__restrict__ ja,
                                                    const double *__restrict__ a,
                                                    const double *__restrict__ thr,
@@ -631,8 +648,8 @@ __global__ __launch_bounds__(256) void k_c_lists_t(int n, const int *__restrict_
    const int gshift = (threadIdx.x & 63) & ~(K - 1);
    const unsigned long long gmask = (K == 64) ? ~0ULL : ((1ULL << K) - 1);
    const unsigned long long below = (1ULL << gl) - 1;
-   const long long r_begin = (long long) blockIdx.x * SF_ROWS;
-   const long long r_end = min((long long) n, r_begin + SF_ROWS);
+   const long long r_begin = (long long) blockIdx.x * rpb;
+   const long long r_end = min((long long) n, r_begin + rpb);
    // a row's own operands are loaded one iteration ahead, while the rows
    // before it run
    int n_s = 0, n_e = 0, n_fl = 2, n_so = 0;
@@ -725,10 +742,11 @@ static void c_lists(const Csr &A, const Csr &S, const int *CF, CLists &L, const 
    if (n == 0) { return; }
    const int K = lanes_per_row(A.nnz, n);
    if (thr && flg) {
-      const int nbf = (int) (((long long) n + SF_ROWS - 1) / SF_ROWS);
+      const int rpb = strength_rows(n, K);
+      const int nbf = (int) (((long long) n + rpb - 1) / rpb);
       dispatch_k(K, [&](auto kc) {
          k_c_lists_t<decltype(kc)::value><<<nbf, 256, 0, stream()>>>(
-             n, A.ia, A.ja, A.a, thr, flg, S.ia, CF, L.sc_cnt, L.sc_ja, L.oc_cnt, L.oc);
+             n, rpb, A.ia, A.ja, A.a, thr, flg, S.ia, CF, L.sc_cnt, L.sc_ja, L.oc_cnt, L.oc);
       });
       HX_LAUNCH_CHECK();
       return;

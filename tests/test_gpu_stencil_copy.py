@@ -18,9 +18,10 @@ pytestmark = pytest.mark.gpu
 
 def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False, positive=0.0):
     """Rows diagonal first, then ascending, from (dx, dy, dz) offsets in
-    symmetric pairs; values 'const', 'few' (64 distinct couplings) or 'all'
-    (every coupling its own); missing: share of the pairs left out; positive:
-    share of small couplings of the diagonal's sign."""
+    symmetric pairs; values 'const', 'few' (64 distinct couplings), 'all'
+    (every coupling its own) or 'late' (constant up to row 1000, inside a
+    slice); missing: share of the pairs left out; positive: share of small
+    couplings of the diagonal's sign."""
     import scipy.sparse as sp
     rng = np.random.default_rng(seed)
     n = nx * ny * nz
@@ -35,7 +36,8 @@ def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False,
         i = np.nonzero(ok)[0]
         j = i + (dz * ny + dy) * nx + dx
         v = {"const": np.ones(len(i)), "few": 0.5 + rng.integers(0, 64, len(i)) / 64.0,
-             "all": 0.5 + rng.random(len(i))}[values]
+             "all": 0.5 + rng.random(len(i)),
+             "late": np.where(i >= 1000, 1.0 + i % 5 / 8, 1.0)}[values]
         v = np.where(rng.random(len(i)) < positive, -0.3 * v, v)
         rows += [i, j]
         cols += [j, i]
@@ -43,7 +45,7 @@ def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False,
     off = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))), shape=(n, n))
     off.sort_indices()
     diag = 1e-2 + np.asarray(abs(off).sum(axis=1)).ravel()
-    if values == "const":
+    if values in ("const", "late"):
         diag[:] = diag.max()
     ia = np.zeros(n + 1, np.int32)
     ia[1:] = np.cumsum(np.diff(off.indptr) + 1)
@@ -74,6 +76,7 @@ P33 = [(k, 0, 0) for k in range(-16, 17)]
 CASES = {
     "27_const_ragged": (17, 19, 23, box(), "const", {}),
     "27_few": (21, 16, 17, box(), "few", {}),
+    "27_late": (21, 16, 17, box(), "late", {}),
     "27_all": (19, 17, 16, box(), "all", {}),
     "27_all_missing": (19, 17, 16, box(), "all", {"missing": 0.2}),
     "27_thin": (2, 61, 47, box(), "few", {}),        # offsets of lines and planes overlap
@@ -134,6 +137,7 @@ def test_product_with_dot_matches_the_csr_kernels(hx, oracle):
 INTERP = {
     "27_const": (17, 19, 23, box(), "const", {}),
     "27_few": (21, 16, 17, box(), "few", {}),
+    "27_late": (21, 16, 17, box(), "late", {}),
     "27_all_signs": (19, 17, 16, box(), "all", {"positive": 0.2}),
     "27_missing": (19, 17, 16, box(), "few", {"missing": 0.25}),
     "27_thin": (2, 61, 47, box(), "few", {}),

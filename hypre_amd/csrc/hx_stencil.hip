@@ -447,7 +447,10 @@ bool sten_probe(const Csr &A, Sten &S, int min_rows, hipStream_t s)
    sten_pinned()->ok = 0;
    k_sten_init<<<1, BS, 0, s>>>(S.st);
    HX_LAUNCH_CHECK();
-   const int nb = (int) std::min<long long>(((long long) A.nrows + 255) / 256, 2048);
+   // half of the wave slots: with all of them, the first kernels of the strength
+   // pass waited for the probe's blocks to end (1.9 ms of 27-point 320^3: setup and
+   // solve 224.1 ms, 222.9 now; 7-point of 1.67 M rows 16.03, 15.94)
+   const int nb = (int) std::min<long long>(((long long) A.nrows + 255) / 256, 1024);
    k_sten_probe<<<nb, BS, 0, s>>>(A.nrows, A.ia, A.ja, S.st);
    HX_LAUNCH_CHECK();
    k_sten_table<<<1, ST_SLOTS, 0, s>>>(S.st, A.a, S.head);

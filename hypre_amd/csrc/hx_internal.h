@@ -178,7 +178,7 @@ struct StenHop
 };
 
 // Stencil copy of an operator for the solve phase (hx_stencil.hip): one mask
-// word a row, slices of 64 rows with no values (all equal to the table's), an
+// word a row, slices of 128 rows with no values (all equal to the table's), an
 // 8-bit code an entry and a dictionary of at most 256 values, or full values.
 struct Sten
 {
@@ -189,9 +189,9 @@ struct Sten
    StenHop  *hop = nullptr;
    unsigned *mask = nullptr;      // bit k: the row has step k
    int      *info = nullptr;      // per slice: mode | 4 if all rows have all steps | values << 8
-   unsigned *codes = nullptr;     // four codes a word, word w of 64 rows contiguous
+   unsigned *codes = nullptr;     // four codes a word, word w of 128 rows contiguous
    double   *dict = nullptr;      // 256 values a slice
-   double   *raw = nullptr;       // step k of 64 rows contiguous (only when some slice needs it)
+   double   *raw = nullptr;       // step k of 128 rows contiguous (only when some slice needs it)
    float    *raw32 = nullptr;
    void      free_all();
 };

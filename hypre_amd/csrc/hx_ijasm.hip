@@ -327,14 +327,19 @@ bool ij_assemble_device(const std::vector<IjChunk> &chunks, int ilower, int nrow
    Csr out;
    out.nrows = nrows;
    out.ncols = ncols;
-   out.ia = dalloc_n<int>((size_t) nrows + 1);
    int h = 0;
    try {
+      out.ia = dalloc_n<int>((size_t) nrows + 1);
       out.nnz = exclusive_scan(cnt, out.ia, nrows);
       d2h(&h, bad, sizeof(int));
       if (h == 0) {
          out.ja = dalloc_n<int>((size_t) std::max<long long>(out.nnz, 1));
          out.a = dalloc_n<double>((size_t) std::max<long long>(out.nnz, 1));
+         k_ij_write<<<nb, BS, 0, s>>>(nrows, op_ia, ocol, oval, dpos, swap_diag, out.ia, out.ja, out.a);
+         HX_LAUNCH_CHECK();
+         // an assembled matrix is complete: its arrays are handed out as they
+         // are, and no stream of the caller's is ordered after this one
+         sync();
       }
    } catch (...) {
       out.free_all();
@@ -344,8 +349,6 @@ bool ij_assemble_device(const std::vector<IjChunk> &chunks, int ilower, int nrow
       out.free_all();
       return false;
    }
-   k_ij_write<<<nb, BS, 0, s>>>(nrows, op_ia, ocol, oval, dpos, swap_diag, out.ia, out.ja, out.a);
-   HX_LAUNCH_CHECK();
    A = out;
    return true;
 }

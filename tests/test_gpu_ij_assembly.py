@@ -138,3 +138,38 @@ def test_column_outside_the_range_is_refused(hx):
     with pytest.raises(hx.HypreError) as e:
         assembled(hx, 0, 2999, 0, 2999, [call])
     assert e.value.code & hx.ERROR_GENERIC
+
+
+class DeviceArray:
+    """A device array of the library as torch sees it."""
+
+    def __init__(self, ptr, n, typestr):
+        self.__cuda_array_interface__ = {"shape": (n,), "typestr": typestr, "data": (ptr, False), "version": 2}
+
+
+def test_assembled_arrays_are_complete_on_return(hx):
+    """The device arrays, read at once on a stream of the caller's: torch's
+    stream and the library's are not ordered.  Memory is recycled between the
+    rounds, so each round has values and columns of its own."""
+    import ctypes
+
+    import torch
+    n, m = 400_000, 27
+    for k in range(4):
+        print("[gpu-ij-assembly] complete", k, flush=True)
+        cols = ((np.arange(n)[:, None] + (k + 1) * np.arange(m)) % n).astype(np.int32)
+        vals = np.random.default_rng(k).standard_normal(n * m)
+        want = torch.from_numpy(vals).cuda(), torch.from_numpy(cols.reshape(-1)).cuda()
+        torch.cuda.synchronize()
+        M = hx.IJMatrix(0, n - 1)
+        M.initialize()
+        M.set_values(np.arange(n), np.full(n, m), cols.reshape(-1), vals)     # the diagonal stands first
+        M.assemble()
+        rows, nnz, ja, a = ctypes.c_int(), ctypes.c_int(), ctypes.c_void_p(), ctypes.c_void_p()
+        hx.call("HYPRE_MI355X_ParCSRMatrixGetDevice", M.get_object().h, ctypes.byref(rows), ctypes.byref(nnz),
+                None, ctypes.byref(ja), ctypes.byref(a))
+        assert (rows.value, nnz.value) == (n, n * m)
+        got = [torch.as_tensor(DeviceArray(p.value, n * m, t), device="cuda").clone()
+               for p, t in ((a, "<f8"), (ja, "<i4"))]
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        M.destroy()

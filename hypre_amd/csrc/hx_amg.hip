@@ -1128,13 +1128,15 @@ HYPRE_Int HYPRE_ParCSRPCGSolve(HYPRE_Solver solver, HYPRE_ParCSRMatrix A, HYPRE_
          const DotParts sp = spmv_dot(M, p->d, sv->d, "spmv_A0");
          double dots[3] = {0.0, 0.0, 0.0};
          const bool ahead = own_precond(s);
-         if (!ahead) { dots[2] = dot_sum(sp); }
-         if (ahead || !pcg_alpha_stops(gamma, dots[2], s->skip_break)) {
+         double sdotp = ahead ? 0.0 : dot_sum(sp);
+         if (ahead || !pcg_alpha_stops(gamma, sdotp, s->skip_break)) {
             pcg_update_xr(n, sp, gamma, s->skip_break, d_sdotp, p->d, sv->d, x->d, r->d);
             apply_precond(s, A, r, sv);
             dot2_sums(dot2_parts(n, r->d, sv->d), d_sdotp, dots);
+            // a caller's preconditioner may itself have run PCG, which keeps its
+            // own <s,p> in that word
+            if (ahead) { sdotp = dots[2]; }
          }
-         const double sdotp = dots[2];
          if (sdotp == 0.0) {
             set_error(HYPRE_ERROR_CONV, "Zero sdotp value in PCG");
             if (i == 1) { i_prod = i_prod_0; }

@@ -1,0 +1,52 @@
+"""PCG where an iteration breaks off, and preconditioners of the caller's own.
+
+The step length is formed on the device; an iteration that hypre's pcg.c leaves
+at it must leave x alone, whoever owns the preconditioner.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+PRECOND = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p)
+
+
+def set_precond(hx, pcg, solve):
+    """A preconditioner of the caller's own; keeps the callbacks alive."""
+    pcg.callbacks = PRECOND(solve), PRECOND(lambda *_: 0)
+    hx.call("HYPRE_ParCSRPCGSetPrecond", pcg.h, *(ctypes.cast(c, ctypes.c_void_p) for c in pcg.callbacks), None)
+
+
+def diagonal(hx, d):
+    n = len(d)
+    return hx.ParCSRMatrix.from_csr(np.arange(n + 1), np.arange(n), np.asarray(d, np.float64))
+
+
+def test_a_preconditioner_that_runs_pcg(hx, oracle):
+    """Diagonal scaling, with and without a PCG solve beside it that ends on
+    <s, p> = 0: the outer iteration is the same, bit for bit."""
+    A = hx.ParCSRMatrix.laplacian7(13, 12, 11)
+    n, _ = A.dims()
+    zero, c, y = diagonal(hx, np.zeros(50)), hx.ParVector(50, np.ones(50)), hx.ParVector(50)
+    inner = hx.PCG(None)
+    inner.setup(zero, c, y)
+
+    def solve(inside):
+        b, x = hx.ParVector(n, 2 * oracle.rand_stream(3, n) - 1), hx.ParVector(n)
+        pcg = hx.PCG(None, tol=1e-8)
+        hx.call("HYPRE_ParCSRPCGSetRelChange", pcg.h, 1)
+
+        def apply(_, a, r, z):
+            hx.call("HYPRE_ParCSRDiagScale", None, *map(ctypes.c_void_p, (a, r, z)))
+            if inside:
+                inner.solve(zero, c, y)
+            return 0
+        set_precond(hx, pcg, apply)
+        pcg.setup(A, b, x)
+        pcg.solve(A, b, x)
+        return pcg.num_iterations(), np.array(pcg.history()), x.get()
+    plain, nested = solve(False), solve(True)
+    assert plain[0] == nested[0] > 10
+    assert np.array_equal(plain[1], nested[1]) and np.array_equal(plain[2], nested[2])

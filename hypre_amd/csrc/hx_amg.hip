@@ -80,10 +80,11 @@ int AMGSolver::sweeps(int lev, int k) const
    return prm.num_sweeps[k];
 }
 
-// values: false when only the solve-phase copy's FP32 values are read
+// values: false when only the solve-phase copy's FP32 values are read (cycle32
+// forms them when that changes)
 static void make_fp32_view(const Csr &src, Csr &dst, bool values = true)
 {
-   dst = src;                 // shares index arrays; owns only a32
+   dst = src;                 // shares index arrays and solve-phase copies; owns only a32
    dst.a = nullptr;
    dst.a32 = nullptr;
    if (!values) { return; }
@@ -518,6 +519,14 @@ void AMGSolver::cycle32(const double *f, double *u)
 {
    Range range("AMGCycle");
    const int nl = num_levels;
+   if (!L[0].f32) { fail(HYPRE_ERROR_GENERIC, "FP32 cycle on a hierarchy set up in FP64"); }
+   // sweeps that were chosen after the setup and do not run on the solve-phase
+   // copies need the values that l1-Jacobi levels do without
+   if (prm.relax_type[1] != 18 || prm.relax_type[2] != 18) {
+      for (int l = 0; l < nl - 1; l++) {
+         if (!L[l].A32.a32) { make_fp32_view(L[l].Av, L[l].A32); }
+      }
+   }
    std::vector<float *> cur(nl), spare(nl);
    for (int l = 0; l < nl; l++) { cur[l] = L[l].u32; spare[l] = L[l].ut32; }
    d2f(L[0].A->nrows, f, L[0].f32);

@@ -812,6 +812,7 @@ void spmv32(const Csr &A, float alpha, const float *x, float beta, const float *
 void spmv_zero_relax(const Csr &A, const double *x, double *y, const double *l1, double w,
                      double *u, const char *cls)
 {
+   if (!l1) { fail(HYPRE_ERROR_GENERIC, "l1-Jacobi without l1 norms"); }
    launch_spmv<double, double, false, true>(A, A.a, 1.0, x, 0.0, nullptr, y, nullptr, cls, 8.0, l1,
                                             w, u);
 }
@@ -819,6 +820,7 @@ void spmv_zero_relax(const Csr &A, const double *x, double *y, const double *l1,
 void spmv32_zero_relax(const Csr &A, const float *x, float *y, const float *l1, float w, float *u,
                        const char *cls)
 {
+   if (!l1) { fail(HYPRE_ERROR_GENERIC, "l1-Jacobi without l1 norms"); }
    if (!A.a32) { fail(HYPRE_ERROR_GENERIC, "FP32 values missing"); }
    launch_spmv<float, float, false, true>(A, A.a32, 1.f, x, 0.f, nullptr, y, nullptr, cls, 4.0, l1,
                                           w, u);
@@ -914,6 +916,8 @@ static void launch_relax_l1(const Csr &A, const V *vals, const X *f, const X *u,
                             X *uo, bool zero, const char *cls, double vbytes)
 {
    if (A.nrows <= 0) { return; }
+   if (!l1) { fail(HYPRE_ERROR_GENERIC, "l1-Jacobi without l1 norms"); }
+   if (!zero && !vals && !A.sten && !A.ell) { fail(HYPRE_ERROR_GENERIC, "matrix values missing"); }
    double xs = sizeof(X);
    double bytes = zero ? xs * 3.0 * A.nrows
                        : (double) A.nnz * (4.0 + vbytes) + 4.0 * (A.nrows + 1) + xs * 4.0 * A.nrows;
@@ -965,6 +969,7 @@ template <typename V, typename X>
 static void launch_relax_jac(const Csr &A, const V *vals, const X *f, const X *u, X w, X *uo)
 {
    if (A.nrows <= 0) { return; }
+   if (!vals) { fail(HYPRE_ERROR_GENERIC, "matrix values missing"); }
    int K = pick_k(A.nnz, A.nrows);
    int nb = grid_for_rows(A.nrows, K);
    hipStream_t s = stream();
@@ -1418,6 +1423,7 @@ static void launch_hgs(int type, const Csr &A, const Csr *Arev, int max_row, con
    // 1266-1383 (8/13/14: Skip_diag 0 only without weights)
    const bool skip = l1t ? !ns : true;
    const int mode = (type == 6 || type == 8) ? 2 : (type == 4 || type == 14) ? 1 : 0;
+   if (mode != 1 && !vals) { fail(HYPRE_ERROR_GENERIC, "matrix values missing"); }
    if (l1t && !l1) { fail(HYPRE_ERROR_GENERIC, "hybrid l1 Gauss-Seidel without l1 norms"); }
    if (mode != 0 && (!Arev || Arev->nrows != A.nrows || !rvals)) {
       fail(HYPRE_ERROR_GENERIC, "backward hybrid Gauss-Seidel without the row-reversed matrix");

@@ -1029,7 +1029,7 @@ static bool cycle_writes_all(const PCGSolver *s, int n)
 {
    if (s->precond != HYPRE_BoomerAMGSolve || !s->precond_solver || s->precond_solver->kind != 1) { return false; }
    const auto *g = static_cast<const AMGSolver *>(s->precond_solver);
-   return g->setup_done && g->L[0].A->nrows == n && g->prm.max_iter >= 1 && !(g->prm.tol > 0.) &&
+   return g->setup_done && g->L[0].A->nrows == n && g->prm.max_iter >= 1 && g->prm.tol <= 0. &&
           g->prm.print_level <= 1 && g->prm.logging <= 1;
 }
 
@@ -1037,9 +1037,17 @@ static void apply_precond(PCGSolver *s, HYPRE_ParCSRMatrix A, hypre_ParVector_st
                           hypre_ParVector_struct *out)
 {
    // ClearVector (par_krylov_func.c:260) then the preconditioner
-   if (s->precond && !cycle_writes_all(s, out->n)) { fill(out->n, 0.0, out->d); }
+   const bool whole = cycle_writes_all(s, out->n);
+   if (s->precond && !whole) { fill(out->n, 0.0, out->d); }
    out->all_zeros = true;
-   if (s->precond) {
+   if (whole) {
+      const int before = g_error_flag;
+      g_error_flag = 0;
+      s->precond(s->precond_solver, A, rhs, out);
+      // a cycle that was refused did not write all
+      if (g_error_flag) { fill(out->n, 0.0, out->d); }
+      g_error_flag |= before;
+   } else if (s->precond) {
       s->precond(s->precond_solver, A, rhs, out);
    } else {
       copy(out->n, rhs->d, out->d);         // identity preconditioner

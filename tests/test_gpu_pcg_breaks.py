@@ -50,3 +50,30 @@ def test_a_preconditioner_that_runs_pcg(hx, oracle):
     plain, nested = solve(False), solve(True)
     assert plain[0] == nested[0] > 10
     assert np.array_equal(plain[1], nested[1]) and np.array_equal(plain[2], nested[2])
+
+
+@pytest.mark.parametrize("how", ["refused", "no_cycle"])
+def test_a_cycle_that_does_not_run_gives_zeros(hx, oracle, how):
+    """A BoomerAMG preconditioner that refuses its sweeps, or whose tolerance
+    lets no cycle run, gives zeros: the vectors of an earlier solve do not
+    show, <s, p> is zero and x stays."""
+    A = hx.ParCSRMatrix.laplacian27(20, 21, 22)
+    n, _ = A.dims()
+    b, x = hx.ParVector(n, 2 * oracle.rand_stream(3, n) - 1), hx.ParVector(n)
+    amg = hx.BoomerAMG()
+    pcg = hx.PCG(amg, tol=1e-8)
+    pcg.setup(A, b, x)
+    pcg.solve(A, b, x)
+    assert pcg.num_iterations() > 3
+    start = oracle.rand_stream(5, n)
+    x.set(start)
+    if how == "refused":
+        amg.set(relax_type=14)              # no reversed rows
+        with pytest.raises(hx.HypreError) as e:
+            pcg.solve(A, b, x)
+        assert e.value.code & hx.ERROR_GENERIC and e.value.code & hx.ERROR_CONV
+    else:
+        amg.set(tol=float("nan"))
+        assert pcg.solve(A, b, x) == hx.ERROR_CONV
+    assert pcg.num_iterations() == 1
+    assert np.array_equal(x.get(), start)

@@ -1017,10 +1017,13 @@ HYPRE_Int HYPRE_ParCSRPCGSetup(HYPRE_Solver solver, HYPRE_ParCSRMatrix A, HYPRE_
    });
 }
 
-// the library's own preconditioners do nothing that a caller could see
+// the library's own preconditioners do nothing that a caller could see, unless
+// they print
 static bool own_precond(const PCGSolver *s)
 {
-   return !s->precond || s->precond == HYPRE_BoomerAMGSolve || s->precond == HYPRE_ParCSRDiagScale;
+   if (!s->precond || s->precond == HYPRE_ParCSRDiagScale) { return true; }
+   return s->precond == HYPRE_BoomerAMGSolve && s->precond_solver && s->precond_solver->kind == 1 &&
+          static_cast<const AMGSolver *>(s->precond_solver)->prm.print_level <= 1;
 }
 
 // a BoomerAMG preconditioner whose one cycle from a zero guess writes every

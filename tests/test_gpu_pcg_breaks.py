@@ -77,3 +77,21 @@ def test_a_cycle_that_does_not_run_gives_zeros(hx, oracle, how):
         assert pcg.solve(A, b, x) == hx.ERROR_CONV
     assert pcg.num_iterations() == 1
     assert np.array_equal(x.get(), start)
+
+
+def test_no_cycle_is_printed_for_an_iteration_that_breaks_off(hx, oracle, capfd):
+    """-A with the hierarchy of A: the first step length is negative.  Only the
+    cycle before it prints."""
+    A = hx.ParCSRMatrix.laplacian7(9, 9, 9)
+    h = A.to_host()
+    minus = hx.ParCSRMatrix.from_csr(h.ia, h.ja, -h.a)
+    n = h.nrows
+    b, x = hx.ParVector(n, 2 * oracle.rand_stream(3, n) - 1), hx.ParVector(n)
+    amg = hx.BoomerAMG()
+    pcg = hx.PCG(amg, tol=1e-8)
+    pcg.setup(A, b, x)
+    amg.set(print_level=2)
+    assert pcg.solve(minus, b, x) & hx.ERROR_CONV
+    ctypes.CDLL(None).fflush(None)
+    assert capfd.readouterr().out.count("Average Convergence Factor") == 1
+    assert pcg.num_iterations() == 1 and not x.get().any()

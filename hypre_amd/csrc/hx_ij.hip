@@ -284,21 +284,23 @@ static void ij_stage(hypre_IJMatrix_struct *m, HYPRE_Int nrows, HYPRE_Int *ncols
    if (!cols) { g_error_arg = 5; fail(HYPRE_ERROR_ARG, "NULL cols"); }
    if (!values) { g_error_arg = 6; fail(HYPRE_ERROR_ARG, "NULL values"); }
    std::vector<int> nc = fetch_input<int>(ncols, (size_t) nrows, m->memloc);
-   if (!m->assembled && (int) m->chunks.size() < IJ_CHUNKS - 2) {
-      size_t ops = 0;
-      for (int i = 0; i < nrows; i++) { ops += (size_t) nc[(size_t) i]; }
-      if (ops >= IJ_DEVICE_MIN && ops <= (size_t) INT_MAX) {
-         // a large call goes to the device as it is
-         ensure_init();
-         ij_flush_staged(m);
-         m->chunks.reserve(m->chunks.size() + 1);
-         m->chunks.push_back(ij_chunk(nrows, (long long) ops, rows, ncols, cols, values, nullptr, op));
-         return;
-      }
+   // a negative length has no entries, here as in the loops below
+   size_t total = 0;
+   bool negative = false;
+   for (int i = 0; i < nrows; i++) {
+      total += (size_t) std::max(nc[(size_t) i], 0);
+      negative = negative || nc[(size_t) i] < 0;
+   }
+   if (!m->assembled && !negative && (int) m->chunks.size() < IJ_CHUNKS - 2 && total >= IJ_DEVICE_MIN &&
+       total <= (size_t) INT_MAX) {
+      // a large call goes to the device as it is
+      ensure_init();
+      ij_flush_staged(m);
+      m->chunks.reserve(m->chunks.size() + 1);
+      m->chunks.push_back(ij_chunk(nrows, (long long) total, rows, ncols, cols, values, nullptr, op));
+      return;
    }
    std::vector<int> rw = fetch_input<int>(rows, (size_t) nrows, m->memloc);
-   size_t total = 0;
-   for (int i = 0; i < nrows; i++) { total += (size_t) nc[(size_t) i]; }
    std::vector<int> cl = fetch_input<int>(cols, total, m->memloc);
    std::vector<double> vl = fetch_input<double>(values, total, m->memloc);
    if (m->assembled) {

@@ -173,3 +173,18 @@ def test_assembled_arrays_are_complete_on_return(hx):
                for p, t in ((a, "<f8"), (ja, "<i4"))]
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
         M.destroy()
+
+
+@pytest.mark.parametrize("rows", [3000, 30])
+def test_negative_row_lengths_have_no_entries(hx, rows):
+    """In large calls, whose prefix sums must not run backwards, and small."""
+    rng = np.random.default_rng(11)
+    op, rw, nc, cl, vl = random_call(rng, "add", np.arange(rows), 0, 2999, 27)
+    none = rng.random(rows) < 0.1
+    keep = np.repeat(~none, nc)
+    given = ("add", rw, np.where(none, -rng.integers(1, 9, rows), nc), cl[keep], vl[keep])
+    same = ("add", rw, np.where(none, 0, nc), cl[keep], vl[keep])
+    m = assembled(hx, 0, 2999, 0, 2999, [given, ("set", rw, np.ones(rows, int), rw.astype(np.int32), vl[:rows])])
+    ia, ja, a = serial(0, 2999, 0, [same, ("set", rw, np.ones(rows, int), rw.astype(np.int32), vl[:rows])])
+    G = m.get_object().to_host()
+    assert np.array_equal(G.ia, ia) and np.array_equal(G.ja, ja) and np.array_equal(G.a, a)

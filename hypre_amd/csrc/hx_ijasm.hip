@@ -4,8 +4,8 @@
 // A chunk is one call's arrays (or many small calls' operations, staged on the
 // host), uploaded as they are: segments (row, length) of columns and values.
 // The segments are grouped by row, each row's in call order, their operations
-// laid out row by row, and one wave a row folds repeated columns in call order
-// and finds the diagonal.  Each row's entries, their order and the order of the
+// laid out row by row, and one wave a row (a block where the row is long) folds
+// repeated columns in call order and finds the diagonal.  Each row's entries, their order and the order of the
 // additions are those of the serial assembly on the host.  What bounds it is
 // the upload: of 0.91 ms for 1.76M operations (110,000 rows), 0.66 are the call
 // that brings their 23 MB, 0.25 the kernels and their read-backs; the serial
@@ -21,6 +21,13 @@ constexpr int BS = 256;
 constexpr int WPB = BS / 64;
 
 static int ij_grid(long long n, int per) { return (int) std::max<long long>(1, std::min<long long>((n + per - 1) / per, 8192)); }
+
+// Rows that take a block.  One row of 512 operations beside 40,000 of nine: the
+// whole assembly 0.52 ms with the row on a wave (0.90 where each operation is a
+// segment of its own), 0.46 with it on a block; 4096 operations 8.2 (26.9)
+// against 0.49 (0.65); at 256 there is nothing between the two.
+constexpr int IJ_LONG = 256;
+__device__ __forceinline__ bool ij_long(int segs, int ops) { return segs > IJ_LONG || ops > IJ_LONG; }
 
 // per row: segments and operations (rows outside [lo, lo + nrows) have none)
 __global__ __launch_bounds__(BS) void k_ij_count(int nseg, const int *__restrict__ rows,
@@ -72,7 +79,7 @@ __global__ __launch_bounds__(BS) void k_ij_layout(int nrows, const IjChunks *__r
    for (int r = blockIdx.x * WPB + wv; r < nrows; r += gridDim.x * WPB) {
       const int b = seg_ia[r], ns = seg_ia[r + 1] - b;
       int o = op_ia[r];
-      if (ns == 0) { continue; }
+      if (ns == 0 || ij_long(ns, op_ia[r + 1] - o)) { continue; }
       if (ns > 1) {
          for (int k = lane; k < ns; k += 64) {
             const int me = list[b + k];
@@ -129,6 +136,7 @@ __global__ __launch_bounds__(BS) void k_ij_layout(int nrows, const IjChunks *__r
 // its place and value, later ones overwrite (0) or add (1) in order.  *bad: a
 // column outside [0, ncols).
 __global__ __launch_bounds__(BS) void k_ij_fold(int nrows, int ncols, int jlo, int diag_shift,
+                                                const int *__restrict__ seg_ia,
                                                 const int *__restrict__ op_ia, int *ocol, double *oval,
                                                 const char *__restrict__ oop, int *__restrict__ cnt,
                                                 int *__restrict__ dpos, int *__restrict__ bad)
@@ -136,6 +144,7 @@ __global__ __launch_bounds__(BS) void k_ij_fold(int nrows, int ncols, int jlo, i
    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
    for (int r = blockIdx.x * WPB + wv; r < nrows; r += gridDim.x * WPB) {
       const int b = op_ia[r], m = op_ia[r + 1] - b;
+      if (ij_long(seg_ia[r + 1] - seg_ia[r], m)) { continue; }
       int have = 0;
       for (int k0 = 0; k0 < m; k0 += 64) {
          const bool act = k0 + lane < m;
@@ -196,9 +205,30 @@ __global__ __launch_bounds__(BS) void k_ij_fold(int nrows, int ncols, int jlo, i
    }
 }
 
-// the rows into CSR, the diagonal (place dpos) first: the entries before it one
-// on, or, with swap, only the first one to its place
-__global__ __launch_bounds__(BS) void k_ij_write(int nrows, const int *__restrict__ op_ia,
+// entries of a row into CSR by the threads t of nt, the diagonal (place dpos)
+// first: the entries before it one on, or, with swap, only the first one to its
+// place
+__device__ __forceinline__ void ij_write_row(int r, int t, int nt, const int *__restrict__ op_ia,
+                                             const int *__restrict__ ocol, const double *__restrict__ oval,
+                                             const int *__restrict__ dpos, bool swap,
+                                             const int *__restrict__ ia, int *__restrict__ ja,
+                                             double *__restrict__ a)
+{
+   const int b = op_ia[r], o = ia[r], m = ia[r + 1] - o, d = dpos[r];
+   for (int q = t; q < m; q += nt) {
+      int to = q;
+      if (d > 0) {
+         if (q == d) { to = 0; }
+         else if (swap) { to = q == 0 ? d : q; }
+         else if (q < d) { to = q + 1; }
+      }
+      ja[o + to] = ocol[b + q];
+      a[o + to] = oval[b + q];
+   }
+}
+
+__global__ __launch_bounds__(BS) void k_ij_write(int nrows, const int *__restrict__ seg_ia,
+                                                 const int *__restrict__ op_ia,
                                                  const int *__restrict__ ocol,
                                                  const double *__restrict__ oval,
                                                  const int *__restrict__ dpos, bool swap,
@@ -207,17 +237,286 @@ __global__ __launch_bounds__(BS) void k_ij_write(int nrows, const int *__restric
 {
    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
    for (int r = blockIdx.x * WPB + wv; r < nrows; r += gridDim.x * WPB) {
-      const int b = op_ia[r], o = ia[r], m = ia[r + 1] - o, d = dpos[r];
-      for (int q = lane; q < m; q += 64) {
-         int to = q;
-         if (d > 0) {
-            if (q == d) { to = 0; }
-            else if (swap) { to = q == 0 ? d : q; }
-            else if (q < d) { to = q + 1; }
+      if (ij_long(seg_ia[r + 1] - seg_ia[r], op_ia[r + 1] - op_ia[r])) { continue; }
+      ij_write_row(r, lane, 64, op_ia, ocol, oval, dpos, swap, ia, ja, a);
+   }
+}
+
+// ------------------------------------------------------------------ long rows
+// Rows of more than IJ_LONG operations or segments (constraints, mean values)
+// by a block each: the wave kernels above compare a row's segments, and its
+// columns, all with all, 1.1 and 0.46 ns times the square of their number.
+// Here the segments are sorted and the columns found in a hash table: a row of
+// 100,000 columns takes 0.9 ms, 3.9 from single operations (most of it the
+// counters that all of them add to); the serial assembly's whole 1.9M operations
+// took 17 to 18.
+constexpr int BL = 1024;
+
+__global__ __launch_bounds__(BS) void k_ij_long_list(int nrows, const int *__restrict__ seg_ia,
+                                                     const int *__restrict__ op_ia, int *__restrict__ rows,
+                                                     int *__restrict__ count)
+{
+   for (int r = blockIdx.x * BS + threadIdx.x; r < nrows; r += gridDim.x * BS) {
+      if (ij_long(seg_ia[r + 1] - seg_ia[r], op_ia[r + 1] - op_ia[r])) { rows[atomicAdd(count, 1)] = r; }
+   }
+}
+
+// exclusive prefix sum over the block (wsum: a word a wave); *total: all of it
+__device__ __forceinline__ int block_excl_scan(int v, int *wsum, int *total)
+{
+   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+   int incl = v;
+   for (int d = 1; d < 64; d <<= 1) {
+      const int t = __shfl_up(incl, d, 64);
+      if (lane >= d) { incl += t; }
+   }
+   if (lane == 63) { wsum[wv] = incl; }
+   __syncthreads();
+   int before = 0, all = 0;
+   for (int w = 0; w < BL / 64; w++) {
+      if (w < wv) { before += wsum[w]; }
+      all += wsum[w];
+   }
+   __syncthreads();
+   *total = all;
+   return before + incl - v;
+}
+
+// A row's segments in call order and their operations at the row's place.  Up
+// to IJ_SORT segment numbers are sorted in LDS.  More are marked as bits, 32
+// IJ_SORT numbers at a time, and the bits read off in order: that takes the
+// list once for every such window between its least and largest number.
+constexpr int IJ_SORT = 8192;
+
+__global__ __launch_bounds__(BL) void k_ij_layout_long(int nlong, const int *__restrict__ rows,
+                                                       const IjChunks *__restrict__ Cp,
+                                                       const int *__restrict__ seg_ia,
+                                                       const int *__restrict__ list, int *sorted,
+                                                       const int *__restrict__ op_ia,
+                                                       int *__restrict__ ocol, double *__restrict__ oval,
+                                                       char *__restrict__ oop)
+{
+   __shared__ int buf[IJ_SORT];
+   __shared__ int off[BL], from[BL], seg[BL], wsum[BL / 64];
+   __shared__ char chunk[BL];
+   const int t = threadIdx.x;
+   for (int w = blockIdx.x; w < nlong; w += gridDim.x) {
+      const int r = rows[w], b = seg_ia[r], ns = seg_ia[r + 1] - b;
+      if (ns <= IJ_SORT) {
+         int n2 = 2;
+         while (n2 < ns) { n2 <<= 1; }
+         for (int k = t; k < n2; k += BL) { buf[k] = k < ns ? list[b + k] : INT_MAX; }
+         __syncthreads();
+         for (int size = 2; size <= n2; size <<= 1) {
+            for (int d = size >> 1; d > 0; d >>= 1) {
+               for (int k = t; k < n2 / 2; k += BL) {
+                  const int i = 2 * k - (k & (d - 1)), j = i + d;
+                  const int x = buf[i], y = buf[j];
+                  if ((x > y) == ((i & size) == 0)) {
+                     buf[i] = y;
+                     buf[j] = x;
+                  }
+               }
+               __syncthreads();
+            }
          }
-         ja[o + to] = ocol[b + q];
-         a[o + to] = oval[b + q];
+         for (int k = t; k < ns; k += BL) { sorted[b + k] = buf[k]; }
+         __syncthreads();
+      } else {
+         if (t == 0) {
+            off[0] = INT_MAX;
+            off[1] = -1;
+         }
+         __syncthreads();
+         int lo = INT_MAX, hi = -1;
+         for (int k = t; k < ns; k += BL) {
+            lo = min(lo, list[b + k]);
+            hi = max(hi, list[b + k]);
+         }
+         atomicMin(off, lo);
+         atomicMax(off + 1, hi);
+         __syncthreads();
+         lo = off[0];
+         hi = off[1];
+         int put = b;
+         constexpr int PER = IJ_SORT / BL;
+         for (long long base = lo; base <= hi; base += 32LL * IJ_SORT) {
+            for (int k = t; k < IJ_SORT; k += BL) { buf[k] = 0; }
+            __syncthreads();
+            for (int k = t; k < ns; k += BL) {
+               const long long g = list[b + k] - base;
+               if (g >= 0 && g < 32LL * IJ_SORT) { atomicOr(buf + (g >> 5), 1 << (g & 31)); }
+            }
+            __syncthreads();
+            int mine = 0, all;
+            for (int k = 0; k < PER; k++) { mine += __popc((unsigned) buf[t * PER + k]); }
+            int at = put + block_excl_scan(mine, wsum, &all);
+            for (int k = 0; k < PER; k++) {
+               for (unsigned bits = (unsigned) buf[t * PER + k]; bits; bits &= bits - 1u) {
+                  sorted[at++] = (int) (base + 32 * (t * PER + k) + __ffs((int) bits) - 1);
+               }
+            }
+            put += all;
+            __syncthreads();
+         }
       }
+      int o = op_ia[r];
+      for (int k0 = 0; k0 < ns; k0 += BL) {
+         int len = 0, st = 0, s = 0, ch = 0, all;
+         if (k0 + t < ns) {
+            const int g = sorted[b + k0 + t];
+            while (ch + 1 < Cp->n && g >= Cp->first[ch + 1]) { ch++; }
+            s = g - Cp->first[ch];
+            st = Cp->start[ch] ? Cp->start[ch][s] : s;
+            len = Cp->start[ch] ? Cp->start[ch][s + 1] - st : 1;
+         }
+         const int place = block_excl_scan(len, wsum, &all);
+         off[t] = place;
+         from[t] = st;
+         seg[t] = s;
+         chunk[t] = (char) ch;
+         __syncthreads();
+         for (int q = t; q < all; q += BL) {
+            int j = 0;      // the last segment that starts at or before q
+            for (int d = BL / 2; d > 0; d >>= 1) {
+               if (off[j + d] <= q) { j += d; }
+            }
+            const int c = chunk[j], e = from[j] + q - off[j];
+            ocol[o + q] = Cp->cols[c][e];
+            oval[o + q] = Cp->vals[c][e];
+            oop[o + q] = Cp->ops[c] ? Cp->ops[c][seg[j]] : Cp->op[c];
+         }
+         o += all;
+         __syncthreads();
+      }
+   }
+}
+
+// The table of a row: column and, beside it, first the least operation seen of
+// the column, then its place (never more than that operation).
+struct IjSlot
+{
+   int col, at;
+};
+
+static __host__ __device__ __forceinline__ unsigned long long ij_slots(int m)
+{
+   unsigned long long c = 64;
+   while (c < 2ull * (unsigned) m) { c <<= 1; }
+   return c;
+}
+
+// A row's operations, BL at a time: each finds its column in the table; the
+// columns' first operations, in order, are the entries' places; then repeated
+// columns overwrite or add, one wave after the other.
+__global__ __launch_bounds__(BL) void k_ij_fold_long(int nlong, const int *__restrict__ rows, int ncols, int jlo,
+                                                     int diag_shift, const int *__restrict__ op_ia, int *ocol,
+                                                     double *oval, const char *__restrict__ oop,
+                                                     IjSlot *__restrict__ tables, unsigned long long table_slots,
+                                                     int *__restrict__ cnt, int *__restrict__ dpos,
+                                                     int *__restrict__ bad)
+{
+   __shared__ int wsum[BL / 64];
+   __shared__ int dplace;
+   constexpr int SCOPE = __HIP_MEMORY_SCOPE_WORKGROUP;
+   const int t = threadIdx.x, wv = t >> 6, lane = t & 63;
+   IjSlot *table = tables + blockIdx.x * table_slots;
+   for (int w = blockIdx.x; w < nlong; w += gridDim.x) {
+      const int r = rows[w], b = op_ia[r], m = op_ia[r + 1] - b;
+      const unsigned long long slots = ij_slots(m);
+      for (unsigned long long k = t; k < slots; k += BL) {
+         __hip_atomic_store(&table[k].col, -1, __ATOMIC_RELAXED, SCOPE);
+         __hip_atomic_store(&table[k].at, INT_MAX, __ATOMIC_RELAXED, SCOPE);
+      }
+      if (t == 0) { dplace = -1; }
+      __syncthreads();
+      int have = 0;
+      for (int k0 = 0; k0 < m; k0 += BL) {
+         const int k = k0 + t;
+         bool act = k < m;
+         int c = 0, op = 0;
+         double v = 0.0;
+         IjSlot *e = table;
+         if (act) {
+            c = ocol[b + k] - jlo;
+            v = oval[b + k];
+            op = oop[b + k];
+            if (c < 0 || c >= ncols) {
+               *bad = 1;
+               act = false;
+            }
+         }
+         if (act) {
+            unsigned long long h = ((unsigned long long) (unsigned) c * 0x9e3779b97f4a7c15ull >> 20) & (slots - 1);
+            while (true) {      // at most half of the slots are ever taken
+               int was = -1;
+               if (__hip_atomic_compare_exchange_strong(&table[h].col, &was, c, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                        SCOPE) ||
+                   was == c) {
+                  break;
+               }
+               h = (h + 1) & (slots - 1);
+            }
+            e = table + h;
+            __hip_atomic_fetch_min(&e->at, k, __ATOMIC_RELAXED, SCOPE);
+         }
+         __syncthreads();
+         const bool fresh = act && __hip_atomic_load(&e->at, __ATOMIC_RELAXED, SCOPE) == k;
+         int all;
+         int place = have + block_excl_scan(fresh, wsum, &all);
+         // all operations of the batch are in registers: their room may be used
+         if (fresh) {
+            __hip_atomic_store(&e->at, place, __ATOMIC_RELAXED, SCOPE);
+            ocol[b + place] = c;
+            oval[b + place] = v;
+            if (c == r + diag_shift) { dplace = place; }
+         }
+         have += all;
+         const bool again = act && !fresh;
+         if (__syncthreads_or(again)) {
+            if (again) { place = __hip_atomic_load(&e->at, __ATOMIC_RELAXED, SCOPE); }
+            // the first lane of this wave with the same column
+            int same = lane;
+            const bool any = __any(again);
+            for (int j = 63; any && j >= 0; j--) {
+               const int pj = __shfl(again ? place : -1, j, 64);
+               if (again && pj == place && j < lane) { same = j; }
+            }
+            const bool lead = again && same == lane, twice = __any(again && !lead);
+            for (int turn = 0; turn < BL / 64; turn++) {
+               if (turn == wv && any) {
+                  double acc = 0.0;
+                  if (lead) { acc = op == 0 ? v : oval[b + place] + v; }
+                  for (int j = 0; twice && j < 64; j++) {
+                     const int sj = __shfl(again ? same : -1, j, 64), oj = __shfl(op, j, 64);
+                     const double vj = __shfl(v, j, 64);
+                     if (sj == lane && j != lane) { acc = oj == 0 ? vj : acc + vj; }
+                  }
+                  if (lead) { oval[b + place] = acc; }
+               }
+               __syncthreads();
+            }
+         }
+      }
+      __syncthreads();
+      if (t == 0) {
+         cnt[r] = have;
+         dpos[r] = dplace;
+      }
+      __syncthreads();
+   }
+}
+
+__global__ __launch_bounds__(BL) void k_ij_write_long(int nlong, const int *__restrict__ rows,
+                                                      const int *__restrict__ op_ia,
+                                                      const int *__restrict__ ocol,
+                                                      const double *__restrict__ oval,
+                                                      const int *__restrict__ dpos, bool swap,
+                                                      const int *__restrict__ ia, int *__restrict__ ja,
+                                                      double *__restrict__ a)
+{
+   for (int w = blockIdx.x; w < nlong; w += gridDim.x) {
+      ij_write_row(rows[w], threadIdx.x, BL, op_ia, ocol, oval, dpos, swap, ia, ja, a);
    }
 }
 
@@ -300,8 +599,9 @@ bool ij_assemble_device(const std::vector<IjChunk> &chunks, int ilower, int nrow
       HX_LAUNCH_CHECK();
       first += c.nseg;
    }
-   const int total_seg = (int) exclusive_scan(seg_ia, seg_ia, nrows);
-   const int total_op = (int) exclusive_scan(op_ia, op_ia, nrows);
+   int most_seg = 0, most_op = 0;
+   const int total_seg = (int) exclusive_scan(seg_ia, seg_ia, nrows, &most_seg);
+   const int total_op = (int) exclusive_scan(op_ia, op_ia, nrows, &most_op);
    d2d(fill, seg_ia, sizeof(int) * ((size_t) nrows + 1));
    int *list = ints((size_t) total_seg), *sorted = ints((size_t) total_seg);
    for (int k = 0; k < C.n; k++) {
@@ -314,16 +614,36 @@ bool ij_assemble_device(const std::vector<IjChunk> &chunks, int ilower, int nrow
    held.push_back(oval);
    char *oop = dalloc_n<char>((size_t) std::max(total_op, 1));
    held.push_back(oop);
-   int *bad = device_flags() + 76;
-   dzero(bad, sizeof(int));
+   int *bad = device_flags() + 76, *nlong_dev = device_flags() + 77;
+   dzero(bad, 2 * sizeof(int));
    const int nb = ij_grid(nrows, WPB);
    IjChunks *dC = dalloc_n<IjChunks>(1);
    held.push_back(dC);
    h2d(dC, &C, sizeof(C));
    k_ij_layout<<<nb, BS, 0, s>>>(nrows, dC, seg_ia, list, sorted, op_ia, ocol, oval, oop);
    HX_LAUNCH_CHECK();
-   k_ij_fold<<<nb, BS, 0, s>>>(nrows, ncols, jlower, ilower - jlower, op_ia, ocol, oval, oop, cnt, dpos, bad);
+   k_ij_fold<<<nb, BS, 0, s>>>(nrows, ncols, jlower, ilower - jlower, seg_ia, op_ia, ocol, oval, oop, cnt, dpos,
+                               bad);
    HX_LAUNCH_CHECK();
+   int nlong = 0, *longs = nullptr;
+   if (most_seg > IJ_LONG || most_op > IJ_LONG) {
+      longs = ints((size_t) nrows);
+      k_ij_long_list<<<ij_grid(nrows, BS), BS, 0, s>>>(nrows, seg_ia, op_ia, longs, nlong_dev);
+      HX_LAUNCH_CHECK();
+      d2h(&nlong, nlong_dev, sizeof(int));
+      // a table a block, in all no more than some times the operations' memory
+      const unsigned long long slots = ij_slots(most_op);
+      const int blocks = (int) std::min<unsigned long long>(
+         (unsigned long long) std::min(nlong, 512), std::max<unsigned long long>(4ull * (unsigned) total_op / slots, 1));
+      IjSlot *tables = dalloc_n<IjSlot>((size_t) (slots * (unsigned) blocks));
+      held.push_back(tables);
+      k_ij_layout_long<<<std::min(nlong, 512), BL, 0, s>>>(nlong, longs, dC, seg_ia, list, sorted, op_ia, ocol, oval,
+                                                           oop);
+      HX_LAUNCH_CHECK();
+      k_ij_fold_long<<<blocks, BL, 0, s>>>(nlong, longs, ncols, jlower, ilower - jlower, op_ia, ocol, oval, oop,
+                                           tables, slots, cnt, dpos, bad);
+      HX_LAUNCH_CHECK();
+   }
    Csr out;
    out.nrows = nrows;
    out.ncols = ncols;
@@ -335,8 +655,13 @@ bool ij_assemble_device(const std::vector<IjChunk> &chunks, int ilower, int nrow
       if (h == 0) {
          out.ja = dalloc_n<int>((size_t) std::max<long long>(out.nnz, 1));
          out.a = dalloc_n<double>((size_t) std::max<long long>(out.nnz, 1));
-         k_ij_write<<<nb, BS, 0, s>>>(nrows, op_ia, ocol, oval, dpos, swap_diag, out.ia, out.ja, out.a);
+         k_ij_write<<<nb, BS, 0, s>>>(nrows, seg_ia, op_ia, ocol, oval, dpos, swap_diag, out.ia, out.ja, out.a);
          HX_LAUNCH_CHECK();
+         if (nlong > 0) {
+            k_ij_write_long<<<std::min(nlong, 512), BL, 0, s>>>(nlong, longs, op_ia, ocol, oval, dpos, swap_diag,
+                                                                out.ia, out.ja, out.a);
+            HX_LAUNCH_CHECK();
+         }
          // an assembled matrix is complete: its arrays are handed out as they
          // are, and no stream of the caller's is ordered after this one
          sync();

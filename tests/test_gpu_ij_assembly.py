@@ -188,3 +188,67 @@ def test_negative_row_lengths_have_no_entries(hx, rows):
     ia, ja, a = serial(0, 2999, 0, [same, ("set", rw, np.ones(rows, int), rw.astype(np.int32), vl[:rows])])
     G = m.get_object().to_host()
     assert np.array_equal(G.ia, ia) and np.array_equal(G.ja, ja) and np.array_equal(G.a, a)
+
+
+def long_row_calls(name, rng):
+    """Calls on n rows and columns with one or some long rows."""
+    n, at = 6000, 2500
+    band = (np.arange(n)[:, None] + np.arange(-4, 5)) % n
+    base = ("set", np.arange(n), np.full(n, 9), band.reshape(-1).astype(np.int32), rng.standard_normal(9 * n))
+
+    def row(op, cols, segs=None):
+        segs = np.array([len(cols)]) if segs is None else segs
+        return op, np.full(len(segs), at), segs, np.asarray(cols, np.int32), rng.standard_normal(len(cols))
+    if name == "dense":
+        return n, [base, row("add", rng.permutation(n))]
+    if name == "duplicates":
+        return n, [row("add", rng.integers(0, 1500, 20000)), base, row("set", rng.integers(0, 1500, 900)),
+                   row("add", rng.integers(700, 2200, 20000))]
+    if name == "one_column":
+        return n, [base, row("add", np.full(5000, 7)), row("add", np.full(3000, at), np.ones(3000, int))]
+    if name == "no_diagonal":
+        return n, [("set", *[np.delete(v, at, 0) for v in base[1:3]], np.delete(base[3].reshape(n, 9), at, 0).ravel(),
+                    base[4][9:]), row("set", np.delete(np.arange(n), at)[::-1])]
+    if name == "segments":              # of 0 to 5 operations
+        segs = rng.integers(0, 6, 5000)
+        return n, [base, row("add", rng.integers(0, n, segs.sum()), segs)]
+    if name == "edges":                 # rows of n operations, and as many segments
+        rw, nc = [], []
+        for r, m in enumerate((255, 256, 257, 1023, 1024, 1025, 2049, 4096)):
+            rw += [r] + [100 + r] * m + [200 + r] * (m + 1)
+            nc += [m] + [1] * m + [1] + [0] * m
+        cl = rng.integers(0, 3000, sum(nc))
+        return n, [("add", np.array(rw), np.array(nc), cl.astype(np.int32), rng.standard_normal(len(cl))), base]
+    assert name == "apart"              # many segments, far apart: several windows, cut at all places
+    rw = np.where(rng.random(700_000) < 0.02, at, rng.integers(0, n, 700_000))
+    return n, [("add", rw, np.ones(len(rw), int), rng.integers(0, n, len(rw)).astype(np.int32),
+                rng.standard_normal(len(rw)))]
+
+
+@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("name", ["dense", "duplicates", "one_column", "no_diagonal", "segments", "edges", "apart"])
+def test_long_rows_follow_the_serial_rule(hx, name, swap):
+    """Rows over 256 operations or segments are taken by blocks."""
+    print("[gpu-ij-assembly] long", name, swap, flush=True)
+    n, calls = long_row_calls(name, np.random.default_rng(13))
+    if name == "apart":
+        at = np.nonzero(calls[0][1] == 2500)[0]
+        assert len(at) > 8192 and at[-1] - at[0] > 2 * 262144
+    check(hx, 0, n - 1, 0, n - 1, calls, swap)
+
+
+def test_long_row_by_many_small_calls(hx):
+    rng = np.random.default_rng(17)
+    n = 4000
+    cols = np.concatenate([rng.permutation(n) for _ in range(9)]).astype(np.int32)
+    calls = [("add" if k % 7 else "set", [3 if k % 8 else k % n], [1], cols[k:k + 1], rng.standard_normal(1))
+             for k in range(len(cols))]
+    check(hx, 0, n - 1, 0, n - 1, calls)
+
+
+def test_column_outside_the_range_in_a_long_row_is_refused(hx):
+    n, calls = long_row_calls("dense", np.random.default_rng(19))
+    calls[1][3][4000] = n
+    with pytest.raises(hx.HypreError) as e:
+        assembled(hx, 0, n - 1, 0, n - 1, calls)
+    assert e.value.code & hx.ERROR_GENERIC

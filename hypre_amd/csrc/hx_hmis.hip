@@ -200,21 +200,28 @@ int hmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_ke
    TimedLaunch tl("setup_hmis_first_pass", 0.0);
    // S^T comes from the device, where it takes 0.6 ms (level 0 of 27-point
    // 64^3): on the host it was nearly half of the pass, and clearing vectors for
-   // the copies a part of the rest (all levels of 64^3: 31 to 37 ms -> 22.5)
+   // the copies a part of the rest (all levels of 64^3: 31 to 37 ms -> 22.5).
+   // Where many rows depend on one point the device would sort that point's row
+   // in one lane, which the host's counting sort does not mind.
    Csr ST;
-   transpose(S, ST, false);
-   Raw<int> ia((size_t) n + 1), ja((size_t) S.nnz), tia((size_t) n + 1), tja((size_t) S.nnz), cf((size_t) n);
+   const bool on_device = transpose(S, ST, false, TRANSPOSE_SORT);
+   Raw<int> ia((size_t) n + 1), ja((size_t) S.nnz), cf((size_t) n);
    try {
       d2h(ia.p, S.ia, sizeof(int) * ((size_t) n + 1));
-      d2h(tia.p, ST.ia, sizeof(int) * ((size_t) n + 1));
       d2h(ja.p, S.ja, sizeof(int) * (size_t) S.nnz);
-      d2h(tja.p, ST.ja, sizeof(int) * (size_t) S.nnz);
+      if (on_device) {
+         Raw<int> tia((size_t) n + 1), tja((size_t) S.nnz);
+         d2h(tia.p, ST.ia, sizeof(int) * ((size_t) n + 1));
+         d2h(tja.p, ST.ja, sizeof(int) * (size_t) S.nnz);
+         ST.free_all();
+         rs_first_pass(n, ia.p, ja.p, tia.p, tja.p, cf.p);
+      } else {
+         rs_first_pass_host(n, ia.p, ja.p, cf.p);
+      }
    } catch (...) {
       ST.free_all();
       throw;
    }
-   ST.free_all();
-   rs_first_pass(n, ia.p, ja.p, tia.p, tja.p, cf.p);
    h2d(CF, cf.p, sizeof(int) * (size_t) n);
    return pmis(S, measure_in_dev, CF, measure_keep_dev, st_count, 1);
 }

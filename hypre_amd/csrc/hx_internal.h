@@ -394,8 +394,11 @@ void correct_cf_marker(int n, int *CF, const int *f2c1, const int *CFN);
 // truncated by (trunc_factor, max_elmts) when either is set; CF -3 -> -1
 void mod_multipass_interp(const Csr &A, const Csr &S, int *CF, int nc, double trunc_factor,
                           int max_elmts, Csr &P);
-// R = P^T, rows ascending (values false: the pattern alone)
-void transpose(const Csr &P, Csr &R, bool values = true);
+// R = P^T, rows ascending (values false: the pattern alone).  Rows of R beyond
+// TRANSPOSE_SORT entries are sorted by one lane; with most_row > 0 nothing is
+// built (false) where a row of R has more entries than that.
+constexpr int TRANSPOSE_SORT = 512;
+bool transpose(const Csr &P, Csr &R, bool values = true, int most_row = 0);
 // p_row_bound / a_row_bound: an upper bound of P's / A's row lengths when the
 // caller knows one (truncation to P_max_elmts; the previous product's
 // ac_max_row), else <= 0; ac_max_row, when given, receives Ac's longest row

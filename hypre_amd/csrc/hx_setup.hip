@@ -3977,7 +3977,7 @@ __global__ __launch_bounds__(256) void k_t_fill_h(int n, const int *__restrict__
 // Rows of R hold distinct fine indices: each entry's final place is its rank
 // in the row.  One wave per row, the row staged in LDS; rows longer than the
 // stage are sorted by insertion in lane 0.
-constexpr int TS_MAX = 512;
+constexpr int TS_MAX = TRANSPOSE_SORT;
 
 template <bool VALUES>
 __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__ Ria,
@@ -4050,7 +4050,7 @@ __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__
    }
 }
 
-void transpose(const Csr &P, Csr &R, bool values)
+bool transpose(const Csr &P, Csr &R, bool values, int most_row)
 {
    int n = P.nrows, nc = P.ncols;
    TimedLaunch tl("setup_transpose", 0.0);
@@ -4066,7 +4066,16 @@ void transpose(const Csr &P, Csr &R, bool values)
    const int nbe = (int) std::max<long long>(1, std::min<long long>(nch, 8192));
    if (P.nnz > 0) { k_col_count_h<<<nbe, 256, 0, stream()>>>(P.nnz, P.ja, R.ia); }
    HX_LAUNCH_CHECK();
-   exclusive_scan_nowait(R.ia, R.ia, nc);   // the total is P.nnz
+   if (most_row > 0) {
+      int longest = 0;
+      exclusive_scan(R.ia, R.ia, nc, &longest);
+      if (longest > most_row) {
+         R.free_all();
+         return false;
+      }
+   } else {
+      exclusive_scan_nowait(R.ia, R.ia, nc);   // the total is P.nnz
+   }
    int *fillp = dalloc_n<int>((size_t) nc + 1);
    d2d(fillp, R.ia, sizeof(int) * ((size_t) nc + 1));
    int nb = std::max(1, std::min((n + 255) / 256, 8192));
@@ -4079,6 +4088,7 @@ void transpose(const Csr &P, Csr &R, bool values)
    }
    HX_LAUNCH_CHECK();
    dfree(fillp);
+   return true;
 }
 
 // ================================================================== RAP

@@ -71,3 +71,18 @@ def test_hmis_hierarchy_bit_exact_and_pcg(hx, oracle, gen):
     assert abs(pcg.num_iterations() - it_ref) <= 1
     r = bh - A_or.to_scipy() @ x.get()
     assert np.linalg.norm(r) / np.linalg.norm(bh) < 1e-8
+
+
+def test_points_that_many_rows_depend_on(hx, oracle):
+    """Rows of S^T of 100,000 entries."""
+    n = 300_000
+    say("hubs", n)
+    i = np.arange(n)
+    cols = np.sort(np.stack([i % 3, np.where(i > 2, i - 1, i + 3), np.minimum(i + 1, n - 1)], 1), 1)
+    keep = (cols != i[:, None]) & np.concatenate([np.ones((n, 1), bool), np.diff(cols, axis=1) > 0], 1)
+    ia = np.zeros(n + 1, np.int32)
+    ia[1:] = np.cumsum(keep.sum(1))
+    S = hx.HostCsr(n, n, ia, cols[keep].astype(np.int32), None)
+    cf_r, rounds_r = oracle.hmis(oracle.Csr(n, n, S.ia, S.ja, np.ones(len(S.ja))))
+    cf_g, rounds_g = hx.hmis(S)
+    assert np.array_equal(cf_g, cf_r) and rounds_g == max(rounds_r, 1)

@@ -73,17 +73,26 @@ struct MeasureBuckets
    }
 };
 
-// memory that is not cleared first and comes in large pages where it can
+// Memory that is not cleared first; arrays from RAW_HUGE on come in large pages
+// where they can.  Clearing a large page takes longer than a small level's whole
+// pass: 1000 points 0.43 ms with all arrays in large pages, 0.24 without.
+constexpr size_t RAW_HUGE = 4000000;
+
 template <class T>
 struct Raw
 {
    T *p;
    explicit Raw(size_t n)
    {
-      const size_t page = size_t(2) << 20, bytes = (std::max<size_t>(n, 1) * sizeof(T) + page - 1) / page * page;
-      p = static_cast<T *>(std::aligned_alloc(page, bytes));
+      const size_t page = size_t(2) << 20, want = std::max<size_t>(n, 1) * sizeof(T);
+      if (want < RAW_HUGE) {
+         p = static_cast<T *>(std::malloc(want));
+      } else {
+         const size_t bytes = (want + page - 1) / page * page;
+         p = static_cast<T *>(std::aligned_alloc(page, bytes));
+         if (p) { (void) madvise(p, bytes, MADV_HUGEPAGE); }
+      }
       if (!p) { throw std::bad_alloc(); }
-      (void) madvise(p, bytes, MADV_HUGEPAGE);
    }
    ~Raw() { std::free(p); }
    Raw(const Raw &) = delete;
@@ -96,7 +105,9 @@ struct Raw
 // par_coarsen.c:1060-1391 for one rank, measure_type 0, cut_factor 0.
 // STi, STj: S^T, each row ascending.  The pass follows S and S^T from point to
 // point and each step needs the one before, so it stays on one host thread; a
-// point is one 16-byte record, and rows that come next are asked for ahead.
+// point is one 16-byte record.  AHEAD: rows that come next are asked for early,
+// which gains 2% at 6.6M entries and costs a tenth where the arrays fit the caches.
+template <bool AHEAD>
 static void rs_first_pass(int n, const int *Si, const int *Sj, const int *STi, const int *STj, int *CF)
 {
    Raw<Point> pts((size_t) n);
@@ -136,7 +147,7 @@ static void rs_first_pass(int n, const int *Si, const int *Sj, const int *STi, c
       const int e = Si[p + 1];
       for (int k = Si[p]; k < e; k++) {
          const int q = Sj[k];
-         if (k + 8 < e) { __builtin_prefetch(pt + Sj[k + 8], 1); }
+         if (AHEAD && k + 8 < e) { __builtin_prefetch(pt + Sj[k + 8], 1); }
          if (pt[q].cf != 0) { continue; }
          B.erase(pt[q].measure, q);
          B.push(++pt[q].measure, q);
@@ -150,7 +161,7 @@ static void rs_first_pass(int n, const int *Si, const int *Sj, const int *STi, c
       pt[c].measure = 0;
       --num_left;
       const int e = STi[c + 1];
-      for (int k = STi[c]; k < e; k++) { __builtin_prefetch(Sj + Si[STj[k]]); }
+      for (int k = STi[c]; AHEAD && k < e; k++) { __builtin_prefetch(Sj + Si[STj[k]]); }
       for (int k = STi[c]; k < e; k++) {
          const int nb = STj[k];
          if (pt[nb].cf != 0) { continue; }
@@ -189,7 +200,7 @@ void rs_first_pass_host(int n, const int *Si, const int *Sj, int *CF)
          for (int k = Si[i]; k < Si[i + 1]; k++) { STj[(size_t) pos[Sj[k]]++] = i; }
       }
    }
-   rs_first_pass(n, Si, Sj, STi.data(), STj.p, CF);
+   rs_first_pass<false>(n, Si, Sj, STi.data(), STj.p, CF);
 }
 
 int hmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_keep_dev,
@@ -198,13 +209,15 @@ int hmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_ke
    const int n = S.nrows;
    if (n == 0) { return 0; }
    TimedLaunch tl("setup_hmis_first_pass", 0.0);
-   // S^T comes from the device, where it takes 0.6 ms (level 0 of 27-point
-   // 64^3): on the host it was nearly half of the pass, and clearing vectors for
-   // the copies a part of the rest (all levels of 64^3: 31 to 37 ms -> 22.5).
+   // S^T of large levels comes from the device, whose launches and copies take
+   // some 0.2 ms.  The split of one level, S^T on the host / on the device:
+   // 27-point 40^3 (1.6M entries) 4.1 / 4.0 ms, 64^3 (6.6M) 21.6 / 18.9; 7-point
+   // 48^3 (110,000 points, 0.65M) 3.0 / 3.7, 64^3 (262,000, 1.5M) 11.7 / 9.4;
+   // 100,000 rows at random, 2.3M entries 12.8 / 14.5, 9.4M 47 / 43.
    // Where many rows depend on one point the device would sort that point's row
    // in one lane, which the host's counting sort does not mind.
    Csr ST;
-   const bool on_device = transpose(S, ST, false, TRANSPOSE_SORT);
+   const bool on_device = (S.nnz >= 2500000 || n >= 200000) && transpose(S, ST, false, TRANSPOSE_SORT);
    Raw<int> ia((size_t) n + 1), ja((size_t) S.nnz), cf((size_t) n);
    try {
       d2h(ia.p, S.ia, sizeof(int) * ((size_t) n + 1));
@@ -214,7 +227,7 @@ int hmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_ke
          d2h(tia.p, ST.ia, sizeof(int) * ((size_t) n + 1));
          d2h(tja.p, ST.ja, sizeof(int) * (size_t) S.nnz);
          ST.free_all();
-         rs_first_pass(n, ia.p, ja.p, tia.p, tja.p, cf.p);
+         rs_first_pass<true>(n, ia.p, ja.p, tia.p, tja.p, cf.p);
       } else {
          rs_first_pass_host(n, ia.p, ja.p, cf.p);
       }

@@ -73,12 +73,14 @@ def test_hmis_hierarchy_bit_exact_and_pcg(hx, oracle, gen):
     assert np.linalg.norm(r) / np.linalg.norm(bh) < 1e-8
 
 
-def test_points_that_many_rows_depend_on(hx, oracle):
-    """Rows of S^T of 100,000 entries."""
+@pytest.mark.parametrize("hubs", [3, 600, 4000])
+def test_points_that_many_rows_depend_on(hx, oracle, hubs):
+    """Rows of S^T of 100,000, 500 and 75 entries, on a level large enough for
+    S^T from the device (the first has rows too long for that)."""
     n = 300_000
-    say("hubs", n)
+    say("hubs", n, hubs)
     i = np.arange(n)
-    cols = np.sort(np.stack([i % 3, np.where(i > 2, i - 1, i + 3), np.minimum(i + 1, n - 1)], 1), 1)
+    cols = np.sort(np.stack([i % hubs, np.where(i > 2, i - 1, i + 3), np.minimum(i + 1, n - 1)], 1), 1)
     keep = (cols != i[:, None]) & np.concatenate([np.ones((n, 1), bool), np.diff(cols, axis=1) > 0], 1)
     ia = np.zeros(n + 1, np.int32)
     ia[1:] = np.cumsum(keep.sum(1))

@@ -3986,6 +3986,8 @@ __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__
    __shared__ int sk[TS_MAX];
    __shared__ double sv[TS_MAX];
    const int lane = threadIdx.x;
+   // a pattern may name a column twice in a row: equal entries keep their order
+   auto before = [](int x, int at, int y, int me) { return x < y || (!VALUES && x == y && at < me); };
    // rows of up to 64 entries are held one entry per lane; the next row's
    // bounds and entries are loaded while the current one is ranked
    int b = 0, e = 0, key = 0;
@@ -4010,7 +4012,7 @@ __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__
          wave_sync();
          if (lane < L) {
             int rank = 0;
-            for (int m = 0; m < L; m++) { rank += (sk[m] < ckey) ? 1 : 0; }
+            for (int m = 0; m < L; m++) { rank += before(sk[m], m, ckey, lane) ? 1 : 0; }
             Rj[cb + rank] = ckey;
             if (VALUES) { Ra[cb + rank] = cval; }
          }
@@ -4042,7 +4044,7 @@ __global__ __launch_bounds__(WAVE) void k_t_sort(int nc, const int *__restrict__
       for (int k = lane; k < L; k += WAVE) {
          const int key = sk[k];
          int rank = 0;
-         for (int m = 0; m < L; m++) { rank += (sk[m] < key) ? 1 : 0; }
+         for (int m = 0; m < L; m++) { rank += before(sk[m], m, key, k) ? 1 : 0; }
          Rj[cb + rank] = key;
          if (VALUES) { Ra[cb + rank] = sv[k]; }
       }

@@ -88,3 +88,22 @@ def test_points_that_many_rows_depend_on(hx, oracle, hubs):
     cf_r, rounds_r = oracle.hmis(oracle.Csr(n, n, S.ia, S.ja, np.ones(len(S.ja))))
     cf_g, rounds_g = hx.hmis(S)
     assert np.array_equal(cf_g, cf_r) and rounds_g == max(rounds_r, 1)
+
+
+def test_a_pattern_with_repeated_columns(hx, oracle):
+    """On a small level and on one whose S^T comes from the device; rows of S^T
+    of up to 64 entries, and of more."""
+    for n, m in ((4000, 8), (210_000, 5), (210_000, 3)):
+        say("repeated", n, m)
+        rng = np.random.default_rng(n + m)
+        cols = (np.arange(n)[:, None] + rng.integers(1, 5, (n, m))) % n
+        if m == 3:
+            cols[:, 0] = np.arange(n) // 100 * 100 + 50
+        keep = cols != np.arange(n)[:, None]
+        assert (np.diff(np.sort(cols, 1), axis=1) == 0).any(1).mean() > 0.2
+        ia = np.zeros(n + 1, np.int32)
+        ia[1:] = np.cumsum(keep.sum(1))
+        S = hx.HostCsr(n, n, ia, cols[keep].astype(np.int32), None)
+        cf_r, rounds_r = oracle.hmis(oracle.Csr(n, n, S.ia, S.ja, np.ones(len(S.ja))))
+        cf_g, rounds_g = hx.hmis(S)
+        assert np.array_equal(cf_g, cf_r) and rounds_g == max(rounds_r, 1)

@@ -1159,8 +1159,11 @@ __global__ __launch_bounds__(256) void k_pmis_update(int nw, const int *__restri
 // block with the list in LDS: a round of three kernels and a read-back takes
 // some 23 us whatever its rows, and half of a level's rounds have few.  The
 // passes are those of k_pmis_remove, k_pmis_cf and k_pmis_update, eight lanes a
-// row, with a barrier between; *rounds_out counts them (-1: no end).
-constexpr int PM_FINISH = 1024;
+// row, with a barrier between; *rounds_out counts them (-1: no end).  One block
+// also reads all their entries, so there may be PM_FINISH_NNZ at the mean length:
+// 1000 rows of 24 take 48 us in one block and 79 in separate kernels, of 75 both
+// 78, of 150 116 and 55, of 600 292 and 33.
+constexpr int PM_FINISH = 1024, PM_FINISH_NNZ = 65536;
 
 __global__ __launch_bounds__(PM_FINISH) void k_pmis_finish(int nw, const int *__restrict__ list,
                                                            const int *__restrict__ S_ia,
@@ -1291,7 +1294,7 @@ int pmis(const Csr &S, const double *measure_in_dev, int *CF, double *measure_ke
    const int *list = nullptr;
    int nw = n;
    while (true) {
-      if (nw <= PM_FINISH) {
+      if (nw <= PM_FINISH && (double) nw * (double) S.nnz <= (double) PM_FINISH_NNZ * n) {
          // what is left, in all its rounds, by one block
          k_pmis_finish<<<1, PM_FINISH, 0, st>>>(nw, list, S.ia, S.ja, m, CF,
                                                !(cf_init != 0 && rounds == 0), h);

@@ -143,6 +143,10 @@ void AMGSolver::setup(const Csr &A0)
       if (st.nslices <= 0) { return; }
       side_sync();
       sten_counts(st);
+      if (setup_verbose()) {
+         std::fprintf(stderr, "[hypre_mi355x] stencil copy: %d offsets, %d slices, %d with codes, %d in full\n",
+                      st.tab.D, st.nslices, st.tab.coded, st.tab.raw);
+      }
       if (st.tab.raw > 0 && !st.raw) {
          side_after_main();
          sten_fill_raw(A0, st, p.cycle_fp32 != 0, side_stream());

@@ -229,6 +229,9 @@ void sten_fill(const Csr &A, Sten &S, hipStream_t s);
 // the counts of slices, into S.tab, once s has finished the fill
 void sten_counts(Sten &S);
 void sten_fill_raw(const Csr &A, Sten &S, bool fp32, hipStream_t s);
+// HYPRE_MI355X_VERBOSE=1 prints the form of the stencil copy and how many rows
+// each setup stage hands on
+bool setup_verbose();
 // Per row of A, as step masks: x strong entries (thr, flg as create_s keeps
 // them), y neighbours that are C points, z neighbours with CF -3, w entries of
 // the sign opposite to the diagonal's

@@ -66,8 +66,7 @@ static int launch_blocks(long long work_items)
    return (int) b;
 }
 
-// HYPRE_MI355X_VERBOSE=1 prints how many rows each setup stage hands on
-static bool setup_verbose()
+bool setup_verbose()
 {
    static const bool v = [] {
       const char *e = std::getenv("HYPRE_MI355X_VERBOSE");

@@ -106,10 +106,9 @@ __global__ __launch_bounds__(BS) void k_sten_probe(int n, const int *__restrict_
          bool fresh;
          const int h = sten_insert(key, c - r, &fresh);
          if (h < 0) { fail = true; break; }
-         if (fresh) {
-            rep[h] = q;
-            if (atomicAdd(&count, 1) >= ST_MAX) { fail = true; break; }
-         }
+         // rows ascend: seldom once the block has seen the offset
+         if (q < *(volatile int *) (rep + h)) { atomicMin(rep + h, q); }
+         if (fresh && atomicAdd(&count, 1) >= ST_MAX) { fail = true; break; }
       }
    }
    if (fail) { bad = 1; }
@@ -132,16 +131,28 @@ __global__ __launch_bounds__(BS) void k_sten_probe(int n, const int *__restrict_
    }
 }
 
-// the table: offset 0 first, then ascending, with the value of one entry of
-// each offset (the one whose index was kept; any entry serves)
-__global__ __launch_bounds__(ST_SLOTS) void k_sten_table(const int *__restrict__ st,
+// The table: offset 0 first, then ascending, with the value of one entry of
+// each offset.  Any entry serves, but slices need no values where they have the
+// table's, so it is taken from inside the grid: from the row of the greatest
+// length that is nearest to the middle (among ST_LOOK tiles of rows around it),
+// for offsets that this row has not the offset's first entry.
+constexpr int ST_TABLE = 1024, ST_LOOK = 256;
+
+__global__ __launch_bounds__(ST_TABLE) void k_sten_table(int n, const int *__restrict__ ia,
+                                                         const int *__restrict__ ja,
                                                          const double *__restrict__ a,
+                                                         const int *__restrict__ st,
                                                          StenHead *__restrict__ out)
 {
-   __shared__ int key[ST_SLOTS];
+   __shared__ int key[ST_SLOTS], rep[ST_SLOTS];
+   __shared__ int best;
    const int i = threadIdx.x;
    const bool ok = st[0] == 0 && st[1] >= 1 && st[1] <= ST_MAX;
-   key[i] = st[ST_KEY + i];
+   if (i < ST_SLOTS) {
+      key[i] = st[ST_KEY + i];
+      rep[i] = st[ST_REP + i];
+   }
+   if (i == 0) { best = INT_MAX; }
    __syncthreads();
    if (i < ST_MAX) {
       out->off[i] = 0;
@@ -155,8 +166,24 @@ __global__ __launch_bounds__(ST_SLOTS) void k_sten_table(const int *__restrict__
       out->coded = 0;
       out->hops = 0;
    }
+   if (!ok) { return; }
+   const int mid = n / 2, longest = st[2];
+   for (int t = 0; t < ST_LOOK; t++) {
+      const int d = t * (ST_TABLE / 2) + (i >> 1);
+      const long long r = (i & 1) ? (long long) mid - 1 - d : (long long) mid + d;
+      const bool hit = r >= 0 && r < n && ia[r + 1] - ia[r] == longest;
+      if (hit) { atomicMin(&best, 2 * d + (i & 1)); }
+      if (__syncthreads_or(hit)) { break; }
+   }
+   if (best != INT_MAX && i < longest) {
+      const int r = (best & 1) ? mid - 1 - (best >> 1) : mid + (best >> 1);
+      const int q = ia[r] + i, d = ja[q] - r;
+      for (int j = 0; j < ST_SLOTS; j++) {
+         if (key[j] == d) { rep[j] = q; }
+      }
+   }
    __syncthreads();
-   if (!ok || key[i] == ST_EMPTY) { return; }
+   if (i >= ST_SLOTS || key[i] == ST_EMPTY) { return; }
    int rank = 0;
    for (int j = 0; j < ST_SLOTS; j++) {
       if (j == i || key[j] == ST_EMPTY) { continue; }
@@ -164,7 +191,7 @@ __global__ __launch_bounds__(ST_SLOTS) void k_sten_table(const int *__restrict__
    }
    if (rank < ST_MAX) {
       out->off[rank] = key[i];
-      out->v[rank] = a[st[ST_REP + i]];
+      out->v[rank] = a[rep[i]];
    }
 }
 
@@ -453,7 +480,7 @@ bool sten_probe(const Csr &A, Sten &S, int min_rows, hipStream_t s)
    const int nb = (int) std::min<long long>(((long long) A.nrows + 255) / 256, 1024);
    k_sten_probe<<<nb, BS, 0, s>>>(A.nrows, A.ia, A.ja, S.st);
    HX_LAUNCH_CHECK();
-   k_sten_table<<<1, ST_SLOTS, 0, s>>>(S.st, A.a, S.head);
+   k_sten_table<<<1, ST_TABLE, 0, s>>>(A.nrows, A.ia, A.ja, A.a, S.st, S.head);
    HX_LAUNCH_CHECK();
    k_sten_hop<<<1, ST_MAX * ST_MAX, 0, s>>>(S.head, S.hop);
    HX_LAUNCH_CHECK();

@@ -10,6 +10,11 @@ table sizes with an unrolled kernel (5, 7, 9, 19, 27) and others, at 31 and
 interpolation, which the stencil path forms one lane a row, must be the
 general kernels' bits for every threshold, truncation and sign pattern.
 """
+import os
+import re
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -169,3 +174,40 @@ def test_interpolation_bits_equal_the_general_kernels(hx, name, options):
     assert np.array_equal(P0.ia, P1.ia) and np.array_equal(P0.ja, P1.ja)
     bad = np.nonzero(P0.a.view(np.int64) != P1.a.view(np.int64))[0]
     assert bad.size == 0, f"{bad.size} of {P0.nnz} weights differ, first at {bad[:5]}"
+
+
+def other_diagonal(rows):
+    ia, ja, a = grid_matrix(32, 32, 32, box(), "const")
+    a[ia[:-1][rows]] *= 2
+    return ia, ja, a
+
+
+# name: matrix, slices with codes and with full values
+FORMS = {
+    "27_const": (lambda: grid_matrix(32, 32, 32, box(), "const"), 0, 0),
+    "27_few": (lambda: grid_matrix(32, 32, 32, box(), "few"), 256, 0),
+    # the first and the last plane have another diagonal: values come from inside
+    "first_plane": (lambda: other_diagonal(slice(0, 1024)), 8, 0),
+    "last_plane": (lambda: other_diagonal(slice(31 * 1024, 32 * 1024)), 8, 0),
+}
+
+
+def report_forms():
+    """Sets every matrix of FORMS up; the library reports to stderr."""
+    from hypre_amd import api
+    api.initialize()
+    for name, (matrix, _, _) in FORMS.items():
+        A = api.ParCSRMatrix.from_csr(*matrix())
+        print("[form]", name, file=sys.stderr, flush=True)
+        api.BoomerAMG(max_levels=2).setup(A)
+
+
+def test_form_of_the_slices():
+    """Which slices keep codes and full values, as HYPRE_MI355X_VERBOSE reports."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-c", "import test_gpu_stencil_copy as t; t.report_forms()"],
+                       capture_output=True, text=True, timeout=110, cwd=here,
+                       env=dict(os.environ, HYPRE_MI355X_VERBOSE="1", PYTHONPATH=os.path.dirname(here)))
+    assert r.returncode == 0, r.stderr
+    got = re.findall(r"\[form\] (\w+)\n.*?(\d+) with codes, (\d+) in full", r.stderr)
+    assert got == [(name, str(coded), str(full)) for name, (_, coded, full) in FORMS.items()]

@@ -143,9 +143,14 @@ void AMGSolver::setup(const Csr &A0)
       if (st.nslices <= 0) { return; }
       side_sync();
       sten_counts(st);
+      const bool pays = sten_pays(A0, st);
       if (setup_verbose()) {
-         std::fprintf(stderr, "[hypre_mi355x] stencil copy: %d offsets, %d slices, %d with codes, %d in full\n",
-                      st.tab.D, st.nslices, st.tab.coded, st.tab.raw);
+         std::fprintf(stderr, "[hypre_mi355x] stencil copy: %d offsets, %d slices, %d with codes, %d in full: %s\n",
+                      st.tab.D, st.nslices, st.tab.coded, st.tab.raw, pays ? "kept" : "dropped");
+      }
+      if (!pays) {
+         st.free_all();
+         return;
       }
       if (st.tab.raw > 0 && !st.raw) {
          side_after_main();

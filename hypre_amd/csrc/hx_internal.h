@@ -228,6 +228,9 @@ bool sten_take(Sten &S);
 void sten_fill(const Csr &A, Sten &S, hipStream_t s);
 // the counts of slices, into S.tab, once s has finished the fill
 void sten_counts(Sten &S);
+// whether, with these counts, the copy's products are faster than those of A's
+// sliced-ELL copy or CSR arrays
+bool sten_pays(const Csr &A, const Sten &S);
 void sten_fill_raw(const Csr &A, Sten &S, bool fp32, hipStream_t s);
 // HYPRE_MI355X_VERBOSE=1 prints the form of the stencil copy and how many rows
 // each setup stage hands on

@@ -16,7 +16,8 @@
 // bit.  Measured against the sliced-ELL kernels (product / l1-Jacobi sweep):
 // 27-point 200^3 constant 511 / 535 -> 73 / 88 us, jumping coefficients
 // 513 / 538 -> 107 / 124 us (FP32 sweep 280 -> 88); 7-point 256^3
-// 363 / 421 -> 100 / 132 us (3.4 TB/s of the bytes left).
+// 363 / 421 -> 100 / 132 us (3.4 TB/s of the bytes left).  Where rows have few of
+// the offsets the copy may not pay (sten_pays).
 #include "hx_internal.h"
 
 #include <algorithm>
@@ -518,6 +519,22 @@ void sten_counts(Sten &S)
 {
    S.tab.raw = sten_pinned()->raw;
    S.tab.coded = sten_pinned()->coded;
+}
+
+// A slice takes the same time however many of the offsets its rows have, the
+// other kernels a time that grows with the entries.  In entries a row (of which
+// the other kernels move some 17 G/ms), an offset costs 0.10 in slices without
+// values, 0.13 with codes and 0.55 with full values.  Products of 120^3 rows, the
+// copy's / the others' by entries a row, us: 27 offsets in full 78 / 107 (26.8),
+// 100 (16.5), 62 (11.3), 45 (7.5); 31 offsets without runs in full 99 / 130
+// (30.7), 115 (18.8), 74 (12.9); 7 in full 29 / 40 (7), 33 (4.6), 24 (2.8); 27
+// with codes 31 / 107, 100, 62, 45 and 33 (4.1); 31 with codes 34 / 39 (4.6); 27
+// without values 21 / 33 (4.1).
+bool sten_pays(const Csr &A, const Sten &S)
+{
+   const double bare = S.nslices - S.tab.coded - S.tab.raw;
+   const double cost = S.tab.D * (0.10 * bare + 0.13 * S.tab.coded + 0.55 * S.tab.raw) / S.nslices;
+   return cost <= (double) A.nnz / A.nrows;
 }
 
 void sten_fill_raw(const Csr &A, Sten &S, bool fp32, hipStream_t s)

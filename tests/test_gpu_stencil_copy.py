@@ -84,6 +84,8 @@ CASES = {
     "27_late": (21, 16, 17, box(), "late", {}),
     "27_all": (19, 17, 16, box(), "all", {}),
     "27_all_missing": (19, 17, 16, box(), "all", {"missing": 0.2}),
+    "27_all_few_entries": (19, 17, 16, box(), "all", {"missing": 0.6}),   # the copy does not pay
+    "27_few_few_entries": (19, 17, 16, box(), "few", {"missing": 0.6}),
     "27_thin": (2, 61, 47, box(), "few", {}),        # offsets of lines and planes overlap
     "19_few": (18, 15, 19, P19, "few", {}),
     "19_const": (64, 8, 8, P19, "const", {}),
@@ -182,13 +184,19 @@ def other_diagonal(rows):
     return ia, ja, a
 
 
-# name: matrix, slices with codes and with full values
+# name: matrix, slices with codes and with full values, whether the copy is kept
 FORMS = {
-    "27_const": (lambda: grid_matrix(32, 32, 32, box(), "const"), 0, 0),
-    "27_few": (lambda: grid_matrix(32, 32, 32, box(), "few"), 256, 0),
+    "27_const": (lambda: grid_matrix(32, 32, 32, box(), "const"), 0, 0, "kept"),
+    "27_few": (lambda: grid_matrix(32, 32, 32, box(), "few"), 256, 0, "kept"),
+    "27_all": (lambda: grid_matrix(32, 32, 32, box(), "all"), 0, 256, "kept"),
+    "27_all_many": (lambda: grid_matrix(32, 32, 32, box(), "all", missing=0.3), 0, 256, "kept"),
+    "27_all_half": (lambda: grid_matrix(32, 32, 32, box(), "all", missing=0.5), 0, 256, "dropped"),
+    "27_few_half": (lambda: grid_matrix(32, 32, 32, box(), "few", missing=0.5), 256, 0, "kept"),
+    "27_const_seldom": (lambda: grid_matrix(32, 32, 32, box(), "const", missing=0.9), 0, 0, "kept"),
+    "31_const_hardly": (lambda: grid_matrix(32, 32, 32, P31, "const", missing=0.97), 0, 0, "dropped"),
     # the first and the last plane have another diagonal: values come from inside
-    "first_plane": (lambda: other_diagonal(slice(0, 1024)), 8, 0),
-    "last_plane": (lambda: other_diagonal(slice(31 * 1024, 32 * 1024)), 8, 0),
+    "first_plane": (lambda: other_diagonal(slice(0, 1024)), 8, 0, "kept"),
+    "last_plane": (lambda: other_diagonal(slice(31 * 1024, 32 * 1024)), 8, 0, "kept"),
 }
 
 
@@ -196,7 +204,7 @@ def report_forms():
     """Sets every matrix of FORMS up; the library reports to stderr."""
     from hypre_amd import api
     api.initialize()
-    for name, (matrix, _, _) in FORMS.items():
+    for name, (matrix, *_) in FORMS.items():
         A = api.ParCSRMatrix.from_csr(*matrix())
         print("[form]", name, file=sys.stderr, flush=True)
         api.BoomerAMG(max_levels=2).setup(A)
@@ -209,5 +217,5 @@ def test_form_of_the_slices():
                        capture_output=True, text=True, timeout=110, cwd=here,
                        env=dict(os.environ, HYPRE_MI355X_VERBOSE="1", PYTHONPATH=os.path.dirname(here)))
     assert r.returncode == 0, r.stderr
-    got = re.findall(r"\[form\] (\w+)\n.*?(\d+) with codes, (\d+) in full", r.stderr)
-    assert got == [(name, str(coded), str(full)) for name, (_, coded, full) in FORMS.items()]
+    got = re.findall(r"\[form\] (\w+)\n.*?(\d+) with codes, (\d+) in full: (\w+)", r.stderr)
+    assert got == [(name, *map(str, want)) for name, (_, *want) in FORMS.items()]

@@ -188,10 +188,11 @@ struct Sten
    StenHead *head = nullptr;
    StenHop  *hop = nullptr;
    unsigned *mask = nullptr;      // bit k: the row has step k
-   int      *info = nullptr;      // per slice: mode | 4 if all rows have all steps | values << 8
+   int      *info = nullptr;      // per slice: mode | 4 if all rows have all steps | << 8: the
+                                  // dictionary's values, or the number among the slices in full
    unsigned *codes = nullptr;     // four codes a word, word w of 128 rows contiguous
    double   *dict = nullptr;      // 256 values a slice
-   double   *raw = nullptr;       // step k of 128 rows contiguous (only when some slice needs it)
+   double   *raw = nullptr;       // by that number, step k of 128 rows contiguous
    float    *raw32 = nullptr;
    void      free_all();
 };
@@ -226,7 +227,8 @@ void ell_fill(const Csr &A, Ell &E, bool fp32, hipStream_t s);
 bool sten_probe(const Csr &A, Sten &S, int min_rows, hipStream_t s);
 bool sten_take(Sten &S);
 void sten_fill(const Csr &A, Sten &S, hipStream_t s);
-// the counts of slices, into S.tab, once s has finished the fill
+// the counts of slices, into S.tab, once s has finished the fill; memory for
+// codes that no slice has is given back
 void sten_counts(Sten &S);
 // whether, with these counts, the copy's products are faster than those of A's
 // sliced-ELL copy or CSR arrays

@@ -412,7 +412,33 @@ __global__ __launch_bounds__(64) void k_sten_fill(int n, int ns, StenHead T,
    }
 }
 
-// the values of the slices that keep them in full, step by step
+// Full values are kept for the slices that need them alone, numbered in order
+// (out of order their products take 3% longer); one block, a stretch of slices a
+// thread.
+constexpr int ST_NUMBER = 1024;
+
+__global__ __launch_bounds__(ST_NUMBER) void k_sten_number(int ns, int *__restrict__ info)
+{
+   __shared__ int sum[ST_NUMBER];
+   const int t = threadIdx.x, per = (ns + ST_NUMBER - 1) / ST_NUMBER;
+   const int s0 = (int) min((long long) ns, (long long) t * per), s1 = min(ns, s0 + per);
+   int c = 0;
+   for (int s = s0; s < s1; s++) { c += (info[s] & 3) == ST_RAW; }
+   sum[t] = c;
+   __syncthreads();
+   for (int d = 1; d < ST_NUMBER; d <<= 1) {
+      const int v = t >= d ? sum[t - d] : 0;
+      __syncthreads();
+      sum[t] += v;
+      __syncthreads();
+   }
+   int at = sum[t] - c;
+   for (int s = s0; s < s1; s++) {
+      if ((info[s] & 3) == ST_RAW) { info[s] |= at++ << 8; }
+   }
+}
+
+// the values of those slices, step by step
 __global__ __launch_bounds__(64) void k_sten_raw(int n, int ns, StenHead T,
                                                  const int *__restrict__ ia,
                                                  const int *__restrict__ ja,
@@ -425,7 +451,9 @@ __global__ __launch_bounds__(64) void k_sten_raw(int n, int ns, StenHead T,
    const int lane = threadIdx.x;
    const int D = T.D;
    for (int sl = blockIdx.x; sl < ns; sl += gridDim.x) {
-      if ((info[sl] & 3) != ST_RAW) { continue; }
+      const int in = info[sl];
+      if ((in & 3) != ST_RAW) { continue; }
+      const size_t base = (size_t) (in >> 8) * D;
       for (int h = 0; h < SF_PARTS; h++) {
          const int f = (int) min((long long) n, (long long) sl * ST_ROWS + h * SF_ROWS);
          const int r = f + lane;
@@ -437,7 +465,7 @@ __global__ __launch_bounds__(64) void k_sten_raw(int n, int ns, StenHead T,
             double v = 0.0;
             if (q < e && sj[q] - r == T.off[k]) { v = sa[q++]; }
             if (lane < SF_ROWS) {
-               const size_t at = ((size_t) sl * D + k) * ST_ROWS + h * SF_ROWS + lane;
+               const size_t at = (base + k) * ST_ROWS + h * SF_ROWS + lane;
                raw[at] = v;
                if (raw32) { raw32[at] = (float) v; }
             }
@@ -519,6 +547,13 @@ void sten_counts(Sten &S)
 {
    S.tab.raw = sten_pinned()->raw;
    S.tab.coded = sten_pinned()->coded;
+   if (S.tab.coded == 0) {
+      // no slice reads them
+      dfree(S.codes);
+      dfree(S.dict);
+      S.codes = nullptr;
+      S.dict = nullptr;
+   }
 }
 
 // A slice takes the same time however many of the offsets its rows have, the
@@ -539,9 +574,11 @@ bool sten_pays(const Csr &A, const Sten &S)
 
 void sten_fill_raw(const Csr &A, Sten &S, bool fp32, hipStream_t s)
 {
-   const size_t words = (size_t) S.nslices * ST_ROWS * S.tab.D;
+   const size_t words = (size_t) S.tab.raw * ST_ROWS * S.tab.D;
    S.raw = dalloc_n<double>(words);
    if (fp32) { S.raw32 = dalloc_n<float>(words); }
+   k_sten_number<<<1, ST_NUMBER, 0, s>>>(S.nslices, S.info);
+   HX_LAUNCH_CHECK();
    k_sten_raw<<<std::min(S.nslices, SF_GRID), 64, 0, s>>>(A.nrows, S.nslices, S.tab, A.ia, A.ja, A.a,
                                                           S.info, S.raw, S.raw32);
    HX_LAUNCH_CHECK();
@@ -820,7 +857,7 @@ __device__ __forceinline__ Two<X> sten_slice(int sl, int lane, int n, bool edge,
 {
    const int mode = h.info & 3;
    const long long f = (long long) sl * ST_ROWS;
-   const V *rw = mode == ST_RAW ? raw + (size_t) sl * ST_ROWS * T->D : nullptr;
+   const V *rw = mode == ST_RAW ? raw + (size_t) (h.info >> 8) * ST_ROWS * T->D : nullptr;
    const unsigned *codes = S.codes + (size_t) sl * ((T->D + 3) / 4) * ST_ROWS;
    if (mode == ST_CODES) {
       const int nd = h.info >> 8;
@@ -1016,7 +1053,7 @@ __global__ __launch_bounds__(BS) void k_sten_masks(int n, int ns, StenView S,
          for (int i = lane; i < (info >> 8); i += 64) { sd[i] = S.dict[(size_t) sl * ST_DICT + i]; }
          __builtin_amdgcn_wave_barrier();
       }
-      const double *rw = raw + (size_t) sl * ST_ROWS * D;
+      const double *rw = mode == ST_RAW ? raw + (size_t) (info >> 8) * ST_ROWS * D : nullptr;
       uint4 a = {0u, 0u, 0u, 0u}, b = {0u, 0u, 0u, 0u};
 #pragma unroll 1
       for (int k0 = 0; k0 < D; k0 += 4) {

@@ -24,8 +24,9 @@ pytestmark = pytest.mark.gpu
 def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False, positive=0.0):
     """Rows diagonal first, then ascending, from (dx, dy, dz) offsets in
     symmetric pairs; values 'const', 'few' (64 distinct couplings), 'all'
-    (every coupling its own) or 'late' (constant up to row 1000, inside a
-    slice); missing: share of the pairs left out; positive: share of small
+    (every coupling its own), 'late' (constant up to row 1000, inside a
+    slice) or 'mixed' (few, from a third of the rows on constant, from two
+    thirds on all); missing: share of the pairs left out; positive: share of small
     couplings of the diagonal's sign."""
     import scipy.sparse as sp
     rng = np.random.default_rng(seed)
@@ -42,7 +43,10 @@ def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False,
         j = i + (dz * ny + dy) * nx + dx
         v = {"const": np.ones(len(i)), "few": 0.5 + rng.integers(0, 64, len(i)) / 64.0,
              "all": 0.5 + rng.random(len(i)),
-             "late": np.where(i >= 1000, 1.0 + i % 5 / 8, 1.0)}[values]
+             "late": np.where(i >= 1000, 1.0 + i % 5 / 8, 1.0),
+             "mixed": np.where(i < n // 3, 0.5 + i * 7 % 64 / 64.0,
+                               np.where(i < 2 * n // 3, 1.0, 0.5 + i * 0.618034 % 1.0 + dz / 7 + dy / 77 + dx / 777)),
+             }[values]
         v = np.where(rng.random(len(i)) < positive, -0.3 * v, v)
         rows += [i, j]
         cols += [j, i]
@@ -50,7 +54,7 @@ def grid_matrix(nx, ny, nz, offsets, values, seed=1, missing=0.0, shuffle=False,
     off = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))), shape=(n, n))
     off.sort_indices()
     diag = 1e-2 + np.asarray(abs(off).sum(axis=1)).ravel()
-    if values in ("const", "late"):
+    if values in ("const", "late", "mixed"):
         diag[:] = diag.max()
     ia = np.zeros(n + 1, np.int32)
     ia[1:] = np.cumsum(np.diff(off.indptr) + 1)
@@ -83,6 +87,9 @@ CASES = {
     "27_few": (21, 16, 17, box(), "few", {}),
     "27_late": (21, 16, 17, box(), "late", {}),
     "27_all": (19, 17, 16, box(), "all", {}),
+    "27_mixed": (16, 16, 48, box(), "mixed", {}),
+    "7_mixed": (23, 25, 24, P7, "mixed", {}),
+    "31_mixed": (9001, 1, 1, P31, "mixed", {}),
     "27_all_missing": (19, 17, 16, box(), "all", {"missing": 0.2}),
     "27_all_few_entries": (19, 17, 16, box(), "all", {"missing": 0.6}),   # the copy does not pay
     "27_few_few_entries": (19, 17, 16, box(), "few", {"missing": 0.6}),
@@ -145,6 +152,7 @@ INTERP = {
     "27_const": (17, 19, 23, box(), "const", {}),
     "27_few": (21, 16, 17, box(), "few", {}),
     "27_late": (21, 16, 17, box(), "late", {}),
+    "27_mixed": (16, 16, 48, box(), "mixed", {}),
     "27_all_signs": (19, 17, 16, box(), "all", {"positive": 0.2}),
     "27_missing": (19, 17, 16, box(), "few", {"missing": 0.25}),
     "27_thin": (2, 61, 47, box(), "few", {}),
@@ -189,6 +197,7 @@ FORMS = {
     "27_const": (lambda: grid_matrix(32, 32, 32, box(), "const"), 0, 0, "kept"),
     "27_few": (lambda: grid_matrix(32, 32, 32, box(), "few"), 256, 0, "kept"),
     "27_all": (lambda: grid_matrix(32, 32, 32, box(), "all"), 0, 256, "kept"),
+    "27_mixed": (lambda: grid_matrix(32, 32, 30, box(), "mixed"), 88, 80, "kept"),
     "27_all_many": (lambda: grid_matrix(32, 32, 32, box(), "all", missing=0.3), 0, 256, "kept"),
     "27_all_half": (lambda: grid_matrix(32, 32, 32, box(), "all", missing=0.5), 0, 256, "dropped"),
     "27_few_half": (lambda: grid_matrix(32, 32, 32, box(), "few", missing=0.5), 256, 0, "kept"),

@@ -80,6 +80,10 @@ P7 = P5 + [(0, 0, 1), (0, 0, -1)]
 P9 = [o for o in box() if o[2] == 0]
 P19 = [o for o in box() if sum(map(abs, o)) <= 2]
 P31 = [(k, 0, 0) for k in range(-15, 16)]
+# 31 offsets whose sums are more than 128
+SCATTERED = [(s * x, s * y, s * z) for s in (-1, 1) for x, y, z in
+             ((1, 0, 0), (3, 0, 0), (7, 0, 0), (-9, 1, 0), (0, 1, 0), (4, 1, 0), (0, 3, 0), (2, 5, 0), (-5, 0, 1),
+              (0, 0, 1), (6, 1, 1), (0, 5, 1), (0, 0, 2), (1, -3, 3), (0, 1, 4))] + [(0, 0, 0)]
 P33 = [(k, 0, 0) for k in range(-16, 17)]
 
 CASES = {
@@ -103,6 +107,8 @@ CASES = {
     "5_all": (67, 71, 1, P5, "all", {}),
     "31_few": (4111, 1, 1, P31, "few", {}),
     "31_all_missing": (5003, 1, 1, P31, "all", {"missing": 0.3}),
+    "scattered_all": (17, 19, 16, SCATTERED, "all", {"missing": 0.1}),
+    "scattered_few": (18, 17, 19, SCATTERED, "few", {}),
     "33_all": (4999, 1, 1, P33, "all", {}),           # one offset too many
     "27_unsorted": (17, 17, 17, box(), "few", {"shuffle": True}),
 }
@@ -161,6 +167,10 @@ INTERP = {
     "7_const": (20, 21, 22, P7, "const", {}),
     "7_signs_missing": (33, 13, 14, P7, "few", {"missing": 0.1, "positive": 0.1}),
     "31_all": (5003, 1, 1, P31, "all", {"missing": 0.3}),
+    "scattered_few": (18, 17, 19, SCATTERED, "few", {}),                   # too many sums: general kernels
+    "scattered_signs": (17, 19, 16, SCATTERED, "all", {"missing": 0.2, "positive": 0.1}),
+    "27_half": (19, 17, 16, box(), "all", {"missing": 0.5}),               # a copy for this alone
+    "27_half_signs": (19, 17, 16, box(), "all", {"missing": 0.6, "positive": 0.1}),
 }
 
 
@@ -199,10 +209,12 @@ FORMS = {
     "27_all": (lambda: grid_matrix(32, 32, 32, box(), "all"), 0, 256, "kept"),
     "27_mixed": (lambda: grid_matrix(32, 32, 30, box(), "mixed"), 88, 80, "kept"),
     "27_all_many": (lambda: grid_matrix(32, 32, 32, box(), "all", missing=0.3), 0, 256, "kept"),
-    "27_all_half": (lambda: grid_matrix(32, 32, 32, box(), "all", missing=0.5), 0, 256, "dropped"),
+    "27_all_half": (lambda: grid_matrix(32, 32, 32, box(), "all", missing=0.5), 0, 256, "interpolation"),
+    "31_all_half": (lambda: grid_matrix(32, 32, 32, P31, "all", missing=0.6), 0, 256, "interpolation"),
+    "too_many_sums": (lambda: grid_matrix(32, 32, 32, SCATTERED, "all", missing=0.6), 0, 256, "dropped"),
     "27_few_half": (lambda: grid_matrix(32, 32, 32, box(), "few", missing=0.5), 256, 0, "kept"),
     "27_const_seldom": (lambda: grid_matrix(32, 32, 32, box(), "const", missing=0.9), 0, 0, "kept"),
-    "31_const_hardly": (lambda: grid_matrix(32, 32, 32, P31, "const", missing=0.97), 0, 0, "dropped"),
+    "31_const_hardly": (lambda: grid_matrix(32, 32, 32, P31, "const", missing=0.97), 0, 0, "interpolation"),
     # the first and the last plane have another diagonal: values come from inside
     "first_plane": (lambda: other_diagonal(slice(0, 1024)), 8, 0, "kept"),
     "last_plane": (lambda: other_diagonal(slice(31 * 1024, 32 * 1024)), 8, 0, "kept"),

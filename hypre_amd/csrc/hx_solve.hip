@@ -72,17 +72,26 @@ constexpr int WPB = BS / 64;   // waves per block
 
 // rows per block: one row per lane; fewer for very long rows, so that a lane's
 // serial sum stays short, and on small matrices, where the round trips of one
-// wave are the whole time: down to about 128 entries a block while there are
-// not yet 4096 blocks (half the waves the device holds).  Measured on whole
-// solves, without -> with: one V-cycle on an irregular matrix of 336,000 rows
-// 313 -> 278 us, PCG on 7-point 30^3 1.89 -> 1.64 ms, 117x131x109 6.72 -> 6.18
-// ms, 256^3 57.2 -> 56.3 ms.
+// wave are the whole time and the device has room for 8192 waves.  Halving pays
+// down to 256 entries a block while there are not yet 4096 blocks, on rows of
+// fewer than 16 entries down to 512 and 3072, and down to 128 while there are
+// not yet 1536.  A product, 64 rows a block / this rule, us: 10,000 rows of 50
+// 6.6 / 4.5, 20,000 of 27 6.8 / 4.2, 100,000 of 27 10.2 / 8.6, 150,000 of 10 6.8 /
+// 6.4; where it stops, going on to 128 entries and 4096 blocks: 60,000 of 10 4.1 /
+// 5.8, 100,000 of 5 4.0 / 5.0, 250,000 of 3 4.6 / 5.6.  One V-cycle on an irregular
+// matrix of 336,000 rows 313 -> 278 us, PCG on 7-point 30^3 1.89 -> 1.64 ms,
+// 117x131x109 6.72 -> 6.18 ms, 256^3 57.2 -> 56.3 ms.
 static int pick_rw(long long nnz, int n)
 {
    double avg = n > 0 ? (double) nnz / n : 1.0;
    int rw = 64;
    while (rw > 1 && rw * avg > 4 * SW) { rw >>= 1; }
-   while (rw > 4 && rw * avg > 128.0 && (n + rw - 1) / rw < 4096) { rw >>= 1; }
+   const bool shorts = avg < 16.0;
+   for (; rw > 4; rw >>= 1) {
+      const double entries = rw * avg;
+      const int most = entries > (shorts ? 512.0 : 256.0) ? (shorts ? 3072 : 4096) : entries > 128.0 ? 1536 : 0;
+      if ((n + rw - 1) / rw >= most) { break; }
+   }
    return rw;
 }
 

@@ -559,7 +559,7 @@ void sten_counts(Sten &S)
 // A slice takes the same time however many of the offsets its rows have, the
 // other kernels a time that grows with the entries.  In entries a row (of which
 // the other kernels move some 17 G/ms), an offset costs 0.10 in slices without
-// values, 0.13 with codes and 0.55 with full values.  Products of 120^3 rows, the
+// values, 0.13 with codes and 0.52 with full values.  Products of 120^3 rows, the
 // copy's / the others' by entries a row, us: 27 offsets in full 78 / 107 (26.8),
 // 100 (16.5), 62 (11.3), 45 (7.5); 31 offsets without runs in full 99 / 130
 // (30.7), 115 (18.8), 74 (12.9); 7 in full 29 / 40 (7), 33 (4.6), 24 (2.8); 27
@@ -568,7 +568,7 @@ void sten_counts(Sten &S)
 bool sten_pays(const Csr &A, const Sten &S)
 {
    const double bare = S.nslices - S.tab.coded - S.tab.raw;
-   const double cost = S.tab.D * (0.10 * bare + 0.13 * S.tab.coded + 0.55 * S.tab.raw) / S.nslices;
+   const double cost = S.tab.D * (0.10 * bare + 0.13 * S.tab.coded + 0.52 * S.tab.raw) / S.nslices;
    return cost <= (double) A.nnz / A.nrows;
 }
 

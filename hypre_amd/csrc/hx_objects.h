@@ -85,7 +85,7 @@ struct AMGParams
    int    keep_setup_data = 0;
    int    hgs_parts = 0;         // hybrid GS partitions on every level (the reference's thread count)
    int    hgs_rows = 4;          // else partitions of about this many rows
-   int    solve_format = 1;      // 1: sliced-ELL copies of the level operators where padding allows; 0: CSR
+   int    solve_format = 1;      // 1: stencil or sliced-ELL copies of the level operators where they pay; 0: CSR
    std::vector<double> level_theta, level_omega;
    std::vector<int>    level_sweeps;
 };

@@ -3339,8 +3339,8 @@ __global__ void k_cf_fix(int n, int *CF)
 // the 19 KB of LDS allow.  Measured and dropped: C-hat as a bit set in
 // registers with ranks by population counts (9 waves a CU, four times the
 // instructions a term: 8.3 ms), terms one at a time (8.2 ms).
-// Level 0 of 27-point 200^3, with masks and truncation: 11.2 + 1.9 + 1.4 ms of
-// separate kernels -> 5.0 + 0.3; jumping coefficients 320^3 55 -> 31 ms.
+// Level 0 of 27-point 200^3, with masks and truncation: 11.2 + 1.6 + 1.4 ms of
+// separate kernels -> 5.0 + 0.3; jumping coefficients 320^3 57 -> 31 ms.
 struct ExtpiStenArgs
 {
    int             n, D, hops;

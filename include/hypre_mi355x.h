@@ -44,9 +44,11 @@ HYPRE_Int HYPRE_MI355X_BoomerAMGGetNumLevels(HYPRE_Solver solver, HYPRE_Int *num
  * fewer (down to 8) on levels with fewer than about 128K partitions. */
 HYPRE_Int HYPRE_MI355X_BoomerAMGSetHybridPartitions(HYPRE_Solver solver, HYPRE_Int parts,
                                                     HYPRE_Int rows);
-/* kernels of the solve phase.  1 (default): at setup, a sliced-ELL copy of
- * each level operator (64-row slices, entries column-major, padding at most
- * 25% of the entries, levels of at least 4096 rows) for the SpMV and
+/* kernels of the solve phase.  1 (default): at setup, a copy of each level
+ * operator of at least 4096 rows (sliced ELL: 64-row slices, entries
+ * column-major, padding at most 25% of the entries; for a fine operator that
+ * is a grid stencil a mask of its offsets a row and values only where slices
+ * of 128 rows need them) for the SpMV and
  * l1-Jacobi kernels and PCG's products with the fine operator, and each
  * coarse level's first l1-Jacobi sweep from a zero guess formed by the
  * restriction that produces its right-hand side.  0: CSR kernels and one

@@ -285,11 +285,17 @@ static void ij_stage(hypre_IJMatrix_struct *m, HYPRE_Int nrows, HYPRE_Int *ncols
    if (!values) { g_error_arg = 6; fail(HYPRE_ERROR_ARG, "NULL values"); }
    std::vector<int> nc = fetch_input<int>(ncols, (size_t) nrows, m->memloc);
    // a negative length has no entries, here as in the loops below
+   const int *len = nc.data();
    size_t total = 0;
-   bool negative = false;
+   int signs = 0;
    for (int i = 0; i < nrows; i++) {
-      total += (size_t) std::max(nc[(size_t) i], 0);
-      negative = negative || nc[(size_t) i] < 0;
+      total += (unsigned) len[i];
+      signs |= len[i];
+   }
+   const bool negative = signs < 0;
+   if (negative) {
+      total = 0;
+      for (int i = 0; i < nrows; i++) { total += (size_t) std::max(len[i], 0); }
    }
    if (!m->assembled && !negative && (int) m->chunks.size() < IJ_CHUNKS - 2 && total >= IJ_DEVICE_MIN &&
        total <= (size_t) INT_MAX) {

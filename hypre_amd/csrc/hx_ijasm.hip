@@ -7,9 +7,10 @@
 // laid out row by row, and one wave a row (a block where the row is long) folds
 // repeated columns in call order and finds the diagonal.  Each row's entries, their order and the order of the
 // additions are those of the serial assembly on the host.  What bounds it is
-// the upload: of 0.91 ms for 1.76M operations (110,000 rows), 0.66 are the call
-// that brings their 23 MB, 0.25 the kernels and their read-backs; the serial
-// assembly took 18.3 ms, and 147 ms for 10.8M operations (5.3 now).
+// the upload: of 0.95 ms for 1.75M operations (110,000 rows), 0.65 are the call
+// that brings their 23 MB, 0.3 the kernels, their read-backs and the wait for the
+// last one; the serial assembly took 18.3 ms, and 147 ms for 10.8M operations (6.0
+// now for 11.1M).
 #include "hx_internal.h"
 
 #include <algorithm>
@@ -27,7 +28,10 @@ static int ij_grid(long long n, int per) { return (int) std::max<long long>(1, s
 // segment of its own), 0.46 with it on a block; 4096 operations 8.2 (26.9)
 // against 0.49 (0.65); at 256 there is nothing between the two.
 constexpr int IJ_LONG = 256;
-__device__ __forceinline__ bool ij_long(int segs, int ops) { return segs > IJ_LONG || ops > IJ_LONG; }
+__device__ __forceinline__ bool ij_long(int r, const int *seg_ia, const int *op_ia)
+{
+   return seg_ia[r + 1] - seg_ia[r] > IJ_LONG || op_ia[r + 1] - op_ia[r] > IJ_LONG;
+}
 
 // per row: segments and operations (rows outside [lo, lo + nrows) have none)
 __global__ __launch_bounds__(BS) void k_ij_count(int nseg, const int *__restrict__ rows,
@@ -67,8 +71,9 @@ struct IjChunks
 };
 
 // One wave a row: its segments by rank into call order, and their operations
-// laid out at the row's place.
-__global__ __launch_bounds__(BS) void k_ij_layout(int nrows, const IjChunks *__restrict__ Cp, const int *__restrict__ seg_ia,
+// laid out at the row's place.  longs, here and below: there are rows to leave to
+// blocks (looking at every row's lengths is a tenth of these kernels' time).
+__global__ __launch_bounds__(BS) void k_ij_layout(int nrows, bool longs, const IjChunks *__restrict__ Cp, const int *__restrict__ seg_ia,
                                                   const int *__restrict__ list,
                                                   int *__restrict__ sorted,
                                                   const int *__restrict__ op_ia,
@@ -79,7 +84,7 @@ __global__ __launch_bounds__(BS) void k_ij_layout(int nrows, const IjChunks *__r
    for (int r = blockIdx.x * WPB + wv; r < nrows; r += gridDim.x * WPB) {
       const int b = seg_ia[r], ns = seg_ia[r + 1] - b;
       int o = op_ia[r];
-      if (ns == 0 || ij_long(ns, op_ia[r + 1] - o)) { continue; }
+      if (ns == 0 || (longs && ij_long(r, seg_ia, op_ia))) { continue; }
       if (ns > 1) {
          for (int k = lane; k < ns; k += 64) {
             const int me = list[b + k];
@@ -135,7 +140,7 @@ __global__ __launch_bounds__(BS) void k_ij_layout(int nrows, const IjChunks *__r
 // ahead of the operations they come from).  A column's first operation gives
 // its place and value, later ones overwrite (0) or add (1) in order.  *bad: a
 // column outside [0, ncols).
-__global__ __launch_bounds__(BS) void k_ij_fold(int nrows, int ncols, int jlo, int diag_shift,
+__global__ __launch_bounds__(BS) void k_ij_fold(int nrows, bool longs, int ncols, int jlo, int diag_shift,
                                                 const int *__restrict__ seg_ia,
                                                 const int *__restrict__ op_ia, int *ocol, double *oval,
                                                 const char *__restrict__ oop, int *__restrict__ cnt,
@@ -144,7 +149,7 @@ __global__ __launch_bounds__(BS) void k_ij_fold(int nrows, int ncols, int jlo, i
    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
    for (int r = blockIdx.x * WPB + wv; r < nrows; r += gridDim.x * WPB) {
       const int b = op_ia[r], m = op_ia[r + 1] - b;
-      if (ij_long(seg_ia[r + 1] - seg_ia[r], m)) { continue; }
+      if (longs && ij_long(r, seg_ia, op_ia)) { continue; }
       int have = 0;
       for (int k0 = 0; k0 < m; k0 += 64) {
          const bool act = k0 + lane < m;
@@ -227,7 +232,7 @@ __device__ __forceinline__ void ij_write_row(int r, int t, int nt, const int *__
    }
 }
 
-__global__ __launch_bounds__(BS) void k_ij_write(int nrows, const int *__restrict__ seg_ia,
+__global__ __launch_bounds__(BS) void k_ij_write(int nrows, bool longs, const int *__restrict__ seg_ia,
                                                  const int *__restrict__ op_ia,
                                                  const int *__restrict__ ocol,
                                                  const double *__restrict__ oval,
@@ -237,7 +242,7 @@ __global__ __launch_bounds__(BS) void k_ij_write(int nrows, const int *__restric
 {
    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
    for (int r = blockIdx.x * WPB + wv; r < nrows; r += gridDim.x * WPB) {
-      if (ij_long(seg_ia[r + 1] - seg_ia[r], op_ia[r + 1] - op_ia[r])) { continue; }
+      if (longs && ij_long(r, seg_ia, op_ia)) { continue; }
       ij_write_row(r, lane, 64, op_ia, ocol, oval, dpos, swap, ia, ja, a);
    }
 }
@@ -257,7 +262,7 @@ __global__ __launch_bounds__(BS) void k_ij_long_list(int nrows, const int *__res
                                                      int *__restrict__ count)
 {
    for (int r = blockIdx.x * BS + threadIdx.x; r < nrows; r += gridDim.x * BS) {
-      if (ij_long(seg_ia[r + 1] - seg_ia[r], op_ia[r + 1] - op_ia[r])) { rows[atomicAdd(count, 1)] = r; }
+      if (ij_long(r, seg_ia, op_ia)) { rows[atomicAdd(count, 1)] = r; }
    }
 }
 
@@ -620,13 +625,14 @@ bool ij_assemble_device(const std::vector<IjChunk> &chunks, int ilower, int nrow
    IjChunks *dC = dalloc_n<IjChunks>(1);
    held.push_back(dC);
    h2d(dC, &C, sizeof(C));
-   k_ij_layout<<<nb, BS, 0, s>>>(nrows, dC, seg_ia, list, sorted, op_ia, ocol, oval, oop);
+   const bool some_long = most_seg > IJ_LONG || most_op > IJ_LONG;
+   k_ij_layout<<<nb, BS, 0, s>>>(nrows, some_long, dC, seg_ia, list, sorted, op_ia, ocol, oval, oop);
    HX_LAUNCH_CHECK();
-   k_ij_fold<<<nb, BS, 0, s>>>(nrows, ncols, jlower, ilower - jlower, seg_ia, op_ia, ocol, oval, oop, cnt, dpos,
-                               bad);
+   k_ij_fold<<<nb, BS, 0, s>>>(nrows, some_long, ncols, jlower, ilower - jlower, seg_ia, op_ia, ocol, oval, oop,
+                               cnt, dpos, bad);
    HX_LAUNCH_CHECK();
    int nlong = 0, *longs = nullptr;
-   if (most_seg > IJ_LONG || most_op > IJ_LONG) {
+   if (some_long) {
       longs = ints((size_t) nrows);
       k_ij_long_list<<<ij_grid(nrows, BS), BS, 0, s>>>(nrows, seg_ia, op_ia, longs, nlong_dev);
       HX_LAUNCH_CHECK();
@@ -655,7 +661,7 @@ bool ij_assemble_device(const std::vector<IjChunk> &chunks, int ilower, int nrow
       if (h == 0) {
          out.ja = dalloc_n<int>((size_t) std::max<long long>(out.nnz, 1));
          out.a = dalloc_n<double>((size_t) std::max<long long>(out.nnz, 1));
-         k_ij_write<<<nb, BS, 0, s>>>(nrows, seg_ia, op_ia, ocol, oval, dpos, swap_diag, out.ia, out.ja, out.a);
+         k_ij_write<<<nb, BS, 0, s>>>(nrows, some_long, seg_ia, op_ia, ocol, oval, dpos, swap_diag, out.ia, out.ja, out.a);
          HX_LAUNCH_CHECK();
          if (nlong > 0) {
             k_ij_write_long<<<std::min(nlong, 512), BL, 0, s>>>(nlong, longs, op_ia, ocol, oval, dpos, swap_diag,

@@ -5,12 +5,12 @@
 // host), uploaded as they are: segments (row, length) of columns and values.
 // The segments are grouped by row, each row's in call order, their operations
 // laid out row by row, and one wave a row (a block where the row is long) folds
-// repeated columns in call order and finds the diagonal.  Each row's entries, their order and the order of the
-// additions are those of the serial assembly on the host.  What bounds it is
-// the upload: of 0.95 ms for 1.75M operations (110,000 rows), 0.65 are the call
-// that brings their 23 MB, 0.3 the kernels, their read-backs and the wait for the
-// last one; the serial assembly took 18.3 ms, and 147 ms for 10.8M operations (6.0
-// now for 11.1M).
+// repeated columns in call order and finds the diagonal.  Each row's entries,
+// their order and the order of the additions are those of the serial assembly
+// on the host.  What bounds it is the upload: of 0.95 ms for 1.75M operations
+// (110,000 rows), 0.65 are the call that brings their 23 MB, 0.3 the kernels,
+// their read-backs and the wait for the last one; the serial assembly took 18.3
+// ms, and 147 ms for 10.8M operations (6.0 now for 11.1M).
 #include "hx_internal.h"
 
 #include <algorithm>
